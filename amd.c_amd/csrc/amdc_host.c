@@ -22,6 +22,7 @@
 
 typedef uint32_t u32;
 typedef uint64_t u64;
+typedef uint16_t u16;
 
 /* ---------------------------------------------------------------- errors */
 
@@ -279,11 +280,13 @@ enum {
   K_GEMVK_Q4 = K_GEMVXW_Q4 + 3, /* amdc_gemv_q4_0_k, _xk, amdc_gemv_q4_k_k, _xk */
   K_GEMVSN_Q4 = K_GEMVK_Q4 + 4, /* amdc_gemv_q4_0_n1 .. _n4, amdc_gemv_q4_k_n1 .. _n4 (fused RMSNorm tail) */
   K_GEMV2N = K_GEMVSN_Q4 + 8,   /* amdc_gemv_q8_0_pn, _q6_k_pn */
-  K_GEMMH_M128 = K_GEMV2N + 2,  /* amdc_gemmh_m128_n128 */
-  K_GEMVM8 = K_GEMMH_M128 + 1,  /* amdc_gemv_q8_0_m1, amdc_gemv_q6_k_m1 */
+  K_GEMVM8 = K_GEMV2N + 2,      /* amdc_gemv_q8_0_m1, amdc_gemv_q6_k_m1 */
   K_GEMVS1W = K_GEMVM8 + 2,     /* amdc_gemv_q4_0_s1w, amdc_gemv_q4_k_s1w */
-  K_N = K_GEMVS1W + 2
+  K_GEMMW_PREP = K_GEMVS1W + 2,
+  K_GEMMW, /* amdc_gemmw_q4_0_n128, _n64, _i128, the same of q4_k and q6_k, amdc_gemmw_q8_0_n128, _n64 */
+  K_N = K_GEMMW + 11
 };
+#define GW(s) "amdc_gemmw_" s
 static const char *const kname[K_N] = {
     "amdc_quant_q8",           "amdc_dots_q4_0",          "amdc_dots_q4_k",          "amdc_gemm_q4_k_n128",
     "amdc_gemm_q4_k_n64",      "amdc_gemv_q4_0_p1",       "amdc_gemv_q4_k_p1",       "amdc_probe_read",
@@ -304,8 +307,10 @@ static const char *const kname[K_N] = {
     "amdc_gemv_q4_0_xk",       "amdc_gemv_q4_k_k",        "amdc_gemv_q4_k_xk",
     "amdc_gemv_q4_0_n1",       "amdc_gemv_q4_0_n2",       "amdc_gemv_q4_0_n3",       "amdc_gemv_q4_0_n4",
     "amdc_gemv_q4_k_n1",       "amdc_gemv_q4_k_n2",       "amdc_gemv_q4_k_n3",       "amdc_gemv_q4_k_n4",
-    "amdc_gemv_q8_0_pn",       "amdc_gemv_q6_k_pn",       "amdc_gemmh_m128_n128",
-    "amdc_gemv_q8_0_m1",       "amdc_gemv_q6_k_m1",       "amdc_gemv_q4_0_s1w",      "amdc_gemv_q4_k_s1w"};
+    "amdc_gemv_q8_0_pn",       "amdc_gemv_q6_k_pn",
+    "amdc_gemv_q8_0_m1",       "amdc_gemv_q6_k_m1",       "amdc_gemv_q4_0_s1w",      "amdc_gemv_q4_k_s1w",
+    GW("prep"), GW("q4_0_n128"), GW("q4_0_n64"), GW("q4_0_i128"), GW("q4_k_n128"), GW("q4_k_n64"), GW("q4_k_i128"),
+    GW("q6_k_n128"), GW("q6_k_n64"), GW("q6_k_i128"), GW("q8_0_n128"), GW("q8_0_n64")};
 
 static hipModule_t g_mod;
 static hipFunction_t g_k[K_N];
@@ -1235,7 +1240,88 @@ static int ws_take(size_t n, void **p) {
 static const struct {
   int k;
   u32 mr, nt, threads;
-} gh[3] = {{K_GEMMH_M64_N128, 64, 128, 256}, {K_GEMMH_M64_N64, 64, 64, 256}, {K_GEMMH_M128, 128, 128, 512}};
+} gh[2] = {{K_GEMMH_M64_N128, 64, 128, 256}, {K_GEMMH_M64_N64, 64, 64, 256}};
+
+/* The prefill GEMM on the wide-tile kernels (amdc_gemmw_*): tiles of 128 rows x 128 or 64 tokens, in three
+ * forms: a tile per CU (512 threads, the two halves of the workgroup taking the super-groups in turn) of 128 or
+ * 64 tokens, and two independent 256-thread workgroups of 128 tokens per CU. Their measured cost per form, in
+ * 0.1 us (MI355X, 34816 x 5120, T = 1000, the time of a round of resident workgroups less GW_ROUND): of two
+ * super-groups for the first two forms, of one for the third, by gw_kind. Q8_0 does not take the third form:
+ * its weight planes at 16 bytes a row outweigh it (512 tokens 360 us against 348). */
+enum { GW_J128, GW_J64, GW_I128, GW_FORMS };
+#define GW_ROUND 40u  /* a round of workgroups: first loads, the tile's output */
+#define GW_REDUCE 40u /* the launch of the split sums */
+static const u16 gw_cost[4][GW_FORMS] = {{66, 39, 63}, {66, 46, 63}, {94, 64, 87}, {75, 58, 0}};
+static u32 gw_kind(int kind) { return kind == AMDC_KIND_Q4_0 ? 0u : kind == AMDC_KIND_Q4_K ? 1u : kind == AMDC_KIND_Q6_K ? 2u : 3u; }
+
+typedef struct {
+  u32 form, nfull, ks; /* tiles [0, nfull) over the whole K, the others in ks splits */
+} gw_plan;
+
+/* The form and schedule with the least estimated time: whole rounds of resident workgroups and the rest of the
+ * tiles split in K, or every tile split, so that the last round is filled; a split costs the launch that adds
+ * the partial sums and their traffic (about 8 TB/s, from L2). Measured against the forms at fixed splits (T = 256, us):
+ * 17408 x 5120 Q4_K 97 whole rounds and 16 tiles in 8 splits, 141 unsplit, 133 all in 2; 5120 x 17408 94 all in
+ * 3, 197 unsplit; 4096 x 4096 33 all in 4, 58 unsplit. */
+static gw_plan gw_choose(int kind, u32 rows, u32 ng, u32 T, u32 cus) {
+  gw_plan best = {T <= 64u ? GW_J64 : GW_J128, 0u, 1u};
+  u64 least = ~0ull;
+  for (u32 f = 0; f < GW_FORMS; f++) {
+    const u32 tw = f == GW_J64 ? 64u : 128u, per = f == GW_I128 ? 1u : 2u, np = (ng + per - 1u) / per;
+    const u32 ntt = (T + tw - 1u) / tw, c = gw_cost[gw_kind(kind)][f];
+    const u64 cap = (u64)cus * (f == GW_I128 ? 2u : 1u), tiles = (u64)((rows + 127u) / 128u) * ntt;
+    if (!c || (tw == 128u && T <= 64u) || (f == GW_I128 && ntt < 2u)) continue;
+    for (u32 whole = 0; whole < 2u; whole++) {
+      const u64 nfull = whole ? tiles / cap * cap / ntt * ntt : 0u, tail = tiles - nfull;
+      if (whole && !nfull) break;
+      const u64 first = (nfull + cap - 1u) / cap * (GW_ROUND + (u64)np * c);
+      for (u32 m = 0; m < 4u; m++) { /* unsplit, or the splits that fill half a round, one or two */
+        u64 ks = m == 0u || !tail ? 1u : (m == 1u ? cap / 2u : (m - 1u) * cap) / tail;
+        if (m && (ks < 2u || (f == GW_I128 && !whole))) continue; /* (the third form loses its sharing of the weights in L2 when split) */
+        if (ks > 16u) ks = 16u; /* amdc_gemm_reduce adds at most 16 splits */
+        if (ks > np) ks = np;
+        u64 est = first;
+        if (tail) est += (tail * ks + cap - 1u) / cap * (GW_ROUND + (np + ks - 1u) / ks * c);
+        if (ks > 1u) est += GW_REDUCE + (2u * ks + 1u) * 4u * tail / ntt * 128u * T / 800000u;
+        if (est < least) least = est, best.form = f, best.nfull = ks > 1u ? (u32)nfull : (u32)tiles, best.ks = (u32)ks;
+      }
+    }
+  }
+  return best;
+}
+
+static int gemmw_launch(int kind, const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias,
+                        const float *res, uint32_t T, uint32_t xs, uint32_t ys, uint32_t rs, void *stream) {
+  const u32 ng = amdc_ngroups(nb), cus = g_cus > 0 ? (u32)g_cus : 256u;
+  gw_plan p = gw_choose(kind, rows, ng, T, cus);
+  if (t_ksplit > 0) p.form = T <= 64u ? GW_J64 : GW_J128;
+  const u32 TW = p.form == GW_J64 ? 64u : 128u, ind = p.form == GW_I128;
+  const u32 ntt = (T + TW - 1u) / TW, tiles = (rows + 127u) / 128u * ntt;
+  if (t_ksplit > 0) {
+    const u32 np = ind ? ng : (ng + 1u) / 2u;
+    p.ks = (u32)t_ksplit < np ? (u32)t_ksplit : np, p.nfull = p.ks > 1u ? 0u : tiles; /* (unsplit tiles go to y) */
+  }
+  const int k = K_GEMMW + 3 * (int)gw_kind(kind) + (int)p.form;
+  const u32 r0 = p.nfull / ntt * 128u, trows = rows > r0 ? rows - r0 : 0u; /* the split tail's rows */
+  u32 ord = kind == AMDC_KIND_Q8_0 ? 1u : kind == AMDC_KIND_Q6_K ? 2u : 0u, q4k = kind == AMDC_KIND_Q4_K;
+  /* the image (amdc_gemmw_prep: 4 ng stages per token tile) and the partial sums */
+  const size_t img_b = (size_t)ntt * ng * 4u * (128u * TW + 1024u + (q4k ? 16u * TW : 0u)), part_b = p.ks > 1u ? (size_t)p.ks * T * trows * 4u : 0u;
+  const u64 grid = (u64)p.nfull + (u64)(tiles - p.nfull) * p.ks;
+  if (grid > 0x7FFFFFFFull || (g_ws_fixed && img_b + part_b > g_scratch_bytes)) return -1;
+  uint8_t *ws = NULL;
+  int rc = ws_take(img_b + part_b, (void **)&ws);
+  if (rc) return rc;
+  void *img = ws, *part = p.ks > 1u ? (void *)(ws + img_b) : NULL;
+  void *pa[] = {&xq, &nb, &T, &xs, &img, (void *)&TW, &ord, &q4k};
+  if ((rc = launch(K_GEMMW_PREP, (unsigned)(ng * (ntt * TW / 32u)), 1, 0, stream, pa))) return rc;
+  void *ga[] = {&w, &img, &y, &rows, &nb, &bias, &res, &T, &ys, &rs, &part, &p.nfull, &p.ks};
+  if ((rc = launch_nt(k, (unsigned)grid, 1, ind ? 256u : 512u, 0, stream, ga)) || p.ks == 1u) return rc;
+  const u64 n = (u64)trows * T; /* the tail rows: y, bias and res from row r0 */
+  float *yt = y + r0;
+  const float *bt = bias ? bias + r0 : NULL, *rt = res ? res + r0 : NULL;
+  void *ra[] = {&part, &p.ks, &yt, (void *)&trows, &T, &bt, &rt, &ys, &rs};
+  return launch(K_GEMM_REDUCE, (unsigned)((n + 255u) / 256u), 1, 0, stream, ra);
+}
 
 /* The prefill GEMM on the f16-MFMA kernels (every kind). */
 static int gemm_launch(int kind, const char *op, const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias,
@@ -1253,14 +1339,21 @@ static int gemm_launch(int kind, const char *op, const void *w, const uint8_t *x
     void *args[] = {&w, &xq, &y, &rows, &nb, &bias, &res, &T, &xs, &ys, &rs};
     return launch(n == 128u ? K_GEMM_N128 : K_GEMM_N64, (unsigned)grid, 1, 0, stream, args);
   }
-  /* the f16-MFMA kernel: 128 tokens per workgroup when there are that many */
+  /* the wide-tile kernels, above 2^22 weights times token tiles of 64: below that the 64-row kernels' shorter way to the
+     first product wins (MI355X, us, 64-row / wide: 1000 x 4096 Q4_K T = 33 13.6 / 16.9, 2048 x 2048 Q6_K T = 64
+     16.1 / 19.5, 4096 x 1024 Q8_0 T = 20 12.8 / 14.9; above, 2048 x 4096 Q4_0 T = 33 18.4 / 16.2, 1000 x 8192 Q4_K T = 64
+     19.7 / 19.8, 4096 x 4096 Q4_K T = 33 27.3 / 19.0). Where the wide kernels' image and partial sums do not fit the
+     fixed workspace of amdc_op_gemv_noalloc, the 64-row ones, which need a little less */
+  const int small = (u64)rows * nb * 32u * ((T + 63u) / 64u) <= (1ull << 22);
+  if (t_gemm == 5 || (t_gemm == 0 && !small)) {
+    if ((rc = gemmw_launch(kind, w, xq, y, rows, nb, bias, res, T, xs, ys, rs, stream)) != -1) return rc;
+    rc = AMDC_OK;
+  }
+  /* the 64-row f16-MFMA kernels: 128 tokens per workgroup when there are that many; 64-token tiles for Q4_0 at any
+     T (its 128-token kernel holds 284 VGPRs, one wave per SIMD: measured 150 / 188 TOPS against 140 / 169 on 11008 x
+     4096 / 4096 x 11008, T = 256) */
   const u32 ng = amdc_ngroups(nb), cus = g_cus > 0 ? (u32)g_cus : 256u;
-  /* 64-token tiles for Q4_0 at any T (its 128-token kernel holds 284 VGPRs, one wave per SIMD:
-     measured 150 / 188 TOPS against 140 / 169 on 11008 x 4096 / 4096 x 11008, T = 256) */
-  /* Q4_K with more than 64 tokens: 128-row tiles below 65536 rows (amdc_gemmh_m128_n128 lists the
-     measurements) */
-  int v = t_gemm >= 3 ? t_gemm - 3 : (T > 64u && kind != AMDC_KIND_Q4_0 ? (kind == AMDC_KIND_Q4_K && rows < 65536u ? 2 : 0) : 1);
-  if (v >= 2 && kind != AMDC_KIND_Q4_K) v = 0; /* the 128-row tile is built for Q4_K */
+  const int v = t_gemm == 3 || t_gemm == 4 ? t_gemm - 3 : (T > 64u && kind != AMDC_KIND_Q4_0 && !small ? 0 : 1);
   const int kk = kind == AMDC_KIND_Q8_0 ? (v ? K_GEMMH_Q8_N64 : K_GEMMH_Q8_N128)
                  : kind == AMDC_KIND_Q6_K ? (v ? K_GEMMH_Q6K_N64 : K_GEMMH_Q6K_N128)
                  : kind == AMDC_KIND_Q4_0 ? (v ? K_GEMMH_Q4_N64 : K_GEMMH_Q4_N128)
@@ -1287,9 +1380,11 @@ static int gemm_launch(int kind, const char *op, const void *w, const uint8_t *x
   }
   if (ks > ng) ks = ng;
   if (ks > 16u) ks = 16u; /* amdc_gemm_reduce adds at most 16 splits */
+  const u32 Tp = (T + 127u) / 128u * 128u, K = 32u * nb;
+  /* the fixed workspace: as many splits as their partial sums leave room for */
+  while (g_ws_fixed && ks > 1u && (size_t)Tp * nb * 72u + (size_t)ks * T * (rows - nfull / ntt * gh[v].mr) * 4u > g_scratch_bytes) ks--;
   if (ks == 1u) nfull = tiles;
   const u32 r0 = nfull / ntt * gh[v].mr, trows = rows - r0; /* the split tail's rows */
-  const u32 Tp = (T + 127u) / 128u * 128u, K = 32u * nb;
   const size_t xh_b = (size_t)Tp * K * 2u, sc_b = (size_t)nb * Tp * 4u, part_b = ks > 1u ? (size_t)ks * T * trows * 4u : 0u;
   uint8_t *ws = NULL;
   rc = ws_take(xh_b + 2u * sc_b + part_b, (void **)&ws);

@@ -22,6 +22,9 @@
 //   amdc_q8_prep, amdc_gemmh_m64_n{64,128}, amdc_gemmh_{q4_0,q8_0,q6_k}_m64_n{64,128}
 //                      the prefill chunk GEMM on the f16 MFMA with exact
 //                      integer block sums (ie_gemm_q4kr, ie_gemm_q8r, ie_gemm_q6kr)
+//   amdc_gemmw_prep, amdc_gemmw_{q4_0,q4_k,q6_k,q8_0}_{n128,n64,i128}
+//                      the same contraction in wide wave tiles from images in the LDS (the default above 2^22 weights
+//                      times token tiles)
 //   amdc_gemm_q4_k_n{64,128}
 //                      the same on int8 MFMA (a tuning alternative)
 //   amdc_chain         a list of quantize / decode-GEMV / RMSNorm+Q8 / SwiGLU+Q8
@@ -2321,12 +2324,12 @@ __device__ __forceinline__ void a_frag_q6(u32 w0, u32 w1, u32 hw, u32 h, int sc,
 // whose partial sums go to part[split][t][r - r0] (r0 the tail's first row,
 // row stride rows - r0) for amdc_gemm_reduce to add in split order. nfull is
 // a whole number of row tiles; nfull = 0 splits every tile.
-template <int NJ, int KIND, u32 MW = 2u>
+template <int NJ, int KIND>
 __device__ __forceinline__ void gemmh_body(const uint8_t *__restrict__ W, const _Float16 *__restrict__ xh, const float *__restrict__ DA,
                                            const float *__restrict__ XA, float *__restrict__ y, u32 rows, u32 nb,
                                            const float *__restrict__ bias, const float *__restrict__ res, u32 T, u32 Tp, u32 ys, u32 rs,
                                            float *__restrict__ part, u32 nfull, u32 nsplit) {
-  constexpr u32 NTH = 128u * MW, MR = 32u * MW, NTT = 32u * NJ; // MW waves of 32 rows x 2 of 16 NJ tokens
+  constexpr u32 MW = 2u, NTH = 128u * MW, MR = 32u * MW, NTT = 32u * NJ; // MW waves of 32 rows x 2 of 16 NJ tokens
   constexpr u32 BSTR = 72u; // halves per token per stage: 2 blocks x 32 + 8 of padding
   __shared__ __attribute__((aligned(16))) _Float16 sb[2][NTT * BSTR];
   __shared__ __attribute__((aligned(16))) float sda[2][2][NTT];
@@ -2593,17 +2596,6 @@ GEMMH_KERNEL(amdc_gemmh_q6_k_m64_n128, 4, AMDC_Q6_K)
 GEMMH_KERNEL(amdc_gemmh_q6_k_m64_n64, 2, AMDC_Q6_K)
 GEMMH_KERNEL(amdc_gemmh_q4_0_m64_n128, 4, AMDC_Q4_0)
 GEMMH_KERNEL(amdc_gemmh_q4_0_m64_n64, 2, AMDC_Q4_0)
-// 128-row tiles, 8 waves (4 x 2): the stage's activations in the LDS shared by twice the rows (Q4_K,
-// T > 64, the default below 65536 rows; measured on MI355X, T = 256, us per call with the prep, 64 /
-// 128-row tiles: 5120 x 17408 185.6 / 161.3, 17408 x 5120 161.5 / 158.1, 34816 x 5120 305 / 288, 4096 x
-// 11008 99.2 / 90.2, 6144 x 5120 82.1 / 76.3, 152064 x 5120 1116 / 1161; 128 rows x 64 tokens, 124
-// VGPRs and two workgroups per CU: 170-266 TOPS, slower everywhere)
-extern "C" __global__ __launch_bounds__(512) void amdc_gemmh_m128_n128(const uint8_t *W, const _Float16 *xh, const float *DA, const float *XA,
-                                                                      float *y, u32 rows, u32 nb, const float *bias, const float *res, u32 T,
-                                                                      u32 Tp, u32 ys, u32 rs, float *part, u32 nfull, u32 nsplit) {
-  gemmh_body<4, AMDC_Q4_K, 4u>(W, xh, DA, XA, y, rows, nb, bias, res, T, Tp, ys, rs, part, nfull, nsplit);
-}
-
 // The split-K sums: y[t][r] = the pairwise tree (adjacent splits first, a
 // split past nks counting as +0.0) of part[0][t][r], part[1][t][r], ...,
 // then the epilogue. nks (1..16) is uniform: one branch on it, then nks loads
@@ -2907,6 +2899,481 @@ __device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t rs, __attribut
   const u32 m = __builtin_amdgcn_readfirstlane((u32)(__UINTPTR_TYPE__)d);
   __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m), "v"(voff), "s"(rs) : "memory");
 }
+
+
+// ------------------------------------------------------------------ prefill GEMM, wide wave tiles
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+
+// The image of the activations that amdc_gemmw_* loads straight into the LDS, 1 KB at a time: token tiles
+// of TW (64 or 128) tokens, per tile 4 ceil(nb / 8) stages of two blocks (2q, 2q + 1 of super-group g, in
+// order), per stage gw_stage() bytes:
+//   B operands  2 blocks x TW / 32 token groups x 2 steps x 64 lanes x 16 bytes: lane (token t % 32, half h =
+//               lane / 32) of step s holds 8 activations as f16, in the order of the weights' A operand
+//   d_a         2 blocks x TW f32 (padded to 1 KB)
+//   Q4_K only: d_a asum of the super-group's 8 blocks as three bf16 parts x = x1 + x2 + x3 (exact), for
+//               the min term: TW / 64 of the tile's TW / 16 chunks of 1 KB, chunk (token group, F): lane
+//               (token, h): F = 0: h ? x2 : x1, F = 1: x3 (8 bf16, the 8 blocks). Tiles of 64: stage
+//               q holds chunk (q / 2, q % 2); tiles of 128: stage q holds chunks (q / 2, q % 2) and
+//               (2 + q / 2, q % 2), one for each half of the waves
+// Tokens past T and blocks past nb are zeros.
+__host__ __device__ constexpr u32 gw_xc(bool q4k, u32 TW) { return q4k ? TW / 64u : 0u; }
+__host__ __device__ constexpr u32 gw_stage(bool q4k, u32 TW) { return 128u * TW + 1024u + 1024u * gw_xc(q4k, TW); }
+
+// A workgroup converts 32 tokens x 8 blocks (one super-group), through the LDS: the Q8 rows are read 256
+// contiguous bytes at a time and the image is written 1 KB at a time. ord: the order of the A operand's 8
+// weights for (half h, step s): 0 (Q4_0, Q4_K): bytes j .. j + 3 of the block, j = 8h + 4s: weights j, j + 2,
+// j + 16, j + 18, j + 1, j + 3, j + 17, j + 19; 1 (Q8_0): 16h + 8s ..; 2 (Q6_K): 16s + 8h ..
+extern "C" __global__ __launch_bounds__(256) void amdc_gemmw_prep(const uint8_t *__restrict__ xq, u32 nb, u32 T, u32 xs, uint8_t *__restrict__ img,
+                                                                  u32 TW, u32 ord, u32 q4k) {
+  constexpr u32 STR = 68u; // dwords per token: 64 + 4 of padding
+  __shared__ __attribute__((aligned(16))) u32 sq[32][STR];
+  __shared__ float sx[8][33];
+  const u32 ng = amdc_ngroups(nb), g = blockIdx.x % ng, b0 = g * 8u, t0 = (blockIdx.x / ng) * 32u, tid = threadIdx.x;
+  const u32 tg = t0 % TW / 32u, SB = gw_stage(q4k != 0u, TW);
+  uint8_t *st = img + ((u64)(t0 / TW) * ng + g) * 4u * SB; // the super-group's 4 stages
+#pragma unroll
+  for (u32 c = 0; c < 2u; c++) {
+    const u32 ch = tid + 256u * c, tl = ch >> 4, k = ch & 15u; // 16 chunks of 16 bytes per token
+    u32x4 v = (u32x4)(0u);
+    if (t0 + tl < T && 2u * b0 + k < 2u * nb) v = *(const u32x4 *)(xq + (u64)(t0 + tl) * xs + 32u * b0 + 16u * k);
+    *(u32x4 *)&sq[tl][4u * k] = v;
+  }
+  {
+    const u32 tl = tid & 31u, bl = tid >> 5, b = b0 + bl;
+    float d = 0.0f, x = 0.0f;
+    if (t0 + tl < T && b < nb) {
+      const uint8_t *xt = xq + (u64)(t0 + tl) * xs;
+      d = ((const float *)(xt + 32u * nb))[b];
+      x = d * (float)(int)((const u32 *)(xt + 36u * nb))[b];
+    }
+    *(float *)(st + (bl >> 1) * SB + 128u * TW + 4u * ((bl & 1u) * TW + t0 % TW + tl)) = d;
+    sx[bl][tl] = x;
+  }
+  __syncthreads();
+  const u32 lane = tid & 63u, w = tid >> 6, tl = lane & 31u, h = lane >> 5;
+#pragma unroll
+  for (u32 k = 0; k < 4u; k++) { // wave w: stage w (blocks 2w, 2w + 1)
+    const u32 bb = k >> 1, s = k & 1u, *q = &sq[tl][8u * (2u * w + bb)];
+    u32x4 o;
+    if (ord == 0u) {
+      const u32 lo = q[2u * h + s], hi = q[4u + 2u * h + s];
+#pragma unroll
+      for (u32 e = 0; e < 4u; e++) {
+        const u32 v = (e & 1u) ? hi : lo, sh = 8u * (e >> 1);
+        const _Float16 a = (_Float16)(int)(int8_t)(v >> sh), b = (_Float16)(int)(int8_t)(v >> (sh + 16u));
+        o[e] = (u32)__builtin_bit_cast(unsigned short, a) | ((u32)__builtin_bit_cast(unsigned short, b) << 16);
+      }
+    } else {
+      const u32 i0 = ord == 1u ? 4u * h + 2u * s : 4u * s + 2u * h;
+#pragma unroll
+      for (u32 e = 0; e < 4u; e++) {
+        const u32 v = q[i0 + (e >> 1)], sh = 16u * (e & 1u);
+        const _Float16 a = (_Float16)(int)(int8_t)(v >> sh), b = (_Float16)(int)(int8_t)(v >> (sh + 8u));
+        o[e] = (u32)__builtin_bit_cast(unsigned short, a) | ((u32)__builtin_bit_cast(unsigned short, b) << 16);
+      }
+    }
+    *(u32x4 *)(st + w * SB + bb * 64u * TW + (2u * tg + s) * 1024u + 16u * lane) = o;
+  }
+  if (q4k && w < 2u) { // wave F: the chunk (tg, F) of the min term
+    u32 part[8];
+#pragma unroll
+    for (u32 b = 0; b < 8u; b++) {
+      const float x = sx[b][tl];
+      const u32 x1 = __builtin_bit_cast(u32, x) & 0xFFFF0000u;
+      const float r1 = x - __builtin_bit_cast(float, x1);
+      const u32 x2 = __builtin_bit_cast(u32, r1) & 0xFFFF0000u;
+      const u32 x3 = __builtin_bit_cast(u32, r1 - __builtin_bit_cast(float, x2));
+      part[b] = w ? x3 : h ? x2 : x1;
+    }
+    u32x4 o;
+#pragma unroll
+    for (u32 e = 0; e < 4u; e++) o[e] = (part[2u * e] >> 16) | (part[2u * e + 1u] & 0xFFFF0000u);
+    const u32 q = (TW == 64u ? 2u * tg : (tg & 1u) << 1) + w;
+    *(u32x4 *)(st + q * SB + 128u * TW + 1024u + (TW == 64u ? 0u : 1024u * (tg >> 1)) + 16u * lane) = o;
+  }
+}
+
+// the masks of the Q4 operands, in registers the compiler does not see through: one v_and_or_b32 each
+struct KW {
+  u32 lo, hi, m;
+};
+__device__ __forceinline__ KW kw() {
+  KW k = {0x000F000Fu, 0x00F000F0u, 0x64006400u};
+  __asm__("" : "+s"(k.lo), "+s"(k.hi));
+  __asm__("" : "+v"(k.m));
+  return k;
+}
+__device__ __forceinline__ h2 spl(h2 v, u32 i) { return i ? (h2){v[1], v[1]} : (h2){v[0], v[0]}; }
+// The 8 weights of dword n of a Q4 block as f16, exact: (1024 + q) s + c for the low nibbles, (1024 + 16 q)
+// s16 + c16 for the high ones; Q4_K: s = (sc, sc / 16), c = -1024 s: q sc. Q4_0: s = (1, 1/16), c = (-1032,
+// -72): q - 8.
+__device__ __forceinline__ h8 a_frag_w(u32 n, h2 s, h2 c, const KW &k) {
+  const u32 n8 = n >> 8;
+  h2 p[4];
+  p[0] = __builtin_bit_cast(h2, (n & k.lo) | k.m);
+  p[1] = __builtin_bit_cast(h2, (n & k.hi) | k.m);
+  p[2] = __builtin_bit_cast(h2, (n8 & k.lo) | k.m);
+  p[3] = __builtin_bit_cast(h2, (n8 & k.hi) | k.m);
+#pragma unroll
+  for (u32 i = 0; i < 4u; i++) p[i] = __builtin_elementwise_fma(p[i], spl(s, i & 1u), spl(c, i & 1u));
+  return (h8){p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
+}
+
+// The two operands of 8 Q6_K weights of a half block: hi = (q - 32) (sc >> 4) and lo = (q - 32) (sc & 15) / 16,
+// both exact in f16, hi + lo = (q - 32) sc / 16. q0, q1: the weights' 6-bit bytes; s = (sc >> 4, (sc & 15) / 16).
+__device__ __forceinline__ void a_frag_w6(u32 q0, u32 q1, h2 s, h8 &hi, h8 &lo) {
+  const h2 c = s * (h2){(_Float16)-1056.0f, (_Float16)-1056.0f};
+  h2 p[4], a[4], b[4];
+  nib_to_h(q0, p[0], p[1]);
+  nib_to_h(q1, p[2], p[3]);
+#pragma unroll
+  for (u32 i = 0; i < 4u; i++) a[i] = __builtin_elementwise_fma(p[i], spl(s, 0u), spl(c, 0u)), b[i] = __builtin_elementwise_fma(p[i], spl(s, 1u), spl(c, 1u));
+  hi = (h8){a[0][0], a[0][1], a[1][0], a[1][1], a[2][0], a[2][1], a[3][0], a[3][1]};
+  lo = (h8){b[0][0], b[0][1], b[1][0], b[1][1], b[2][0], b[2][1], b[3][0], b[3][1]};
+}
+
+// Y[t][r], the arguments of gemmh_body, from the image of amdc_gemmw_prep; any kind. Per block b of super-group g
+//   X_rtb = sum_k w_rk a_tk, exact integers on the f16 MFMA (Q4_K: q sc; Q6_K: (q - 32) sc / 16 in two operands;
+//   Q4_0: q - 8; Q8_0: the int8 weight)
+//   Q4_K, Q6_K: tmp_rt += da_tb X_rtb, per super-block acc_rt += d_rg tmp_rt, Q4_K: acc_rt -= sum_b (dmin mn)_rb xa_tb
+//   Q4_0, Q8_0: acc_rt += (d_rb da_tb) X_rtb
+// What bounds it is the issue of vector instructions (4 cycles each, an MFMA 8; measured): one fma per element and
+// block, the A operands, and waits. So:
+// - a wave takes 64 rows x 32 NJ tokens in 32 x 32 tiles: an A operand (9 instructions per 8 weights) serves 64
+//   tokens where gemmh's serves 32, and half as many MFMAs are issued as in 16 x 16 tiles;
+// - everything comes into the LDS by loads that touch no register, a stage of two blocks at a time, a stage or two
+//   ahead, one barrier per stage; the activations as prepared images of it, so that every read of it is 16
+//   consecutive bytes per lane;
+// - the scales are unpacked once per workgroup into tables in the LDS, not by every wave that uses them;
+// - Q4_K's min term runs on the bf16 MFMA as 6 products of exact parts (768 fewer matrix cycles per super-block and
+//   wave than in f32, which took 15 % of the time); Q4_0 / Q8_0's d_w d_a is an outer product on the f32 MFMA
+//   (rank 1, one rounding) instead of a multiply per element and block.
+// GR = 2: one 512-thread workgroup per CU, two groups of 4 waves that take the super-groups of the tile in turn, half a
+// stage apart, and add their sums through the LDS at the end: both waves of a SIMD work on one tile where there are
+// only about as many tiles as CUs. GR = 1: a 256-thread workgroup per tile, two independent ones per CU, whose waits
+// overlap better (34816 x 5120 Q4_K, T = 1024: 617 against 675 us), for matrices of many tiles.
+// Measured on MI355X (us, whole call with the quantization, gemmh / this): 17408 x 5120 Q4_K T = 256 146.8 / 100.1,
+// 34816 x 5120 Q4_K T = 1024 1024 / 628 (582 TOPS), 11008 x 4096 Q4_0 T = 77 93.7 / 43.9, 5120 x 17408 Q6_K T = 256 236 /
+// 150, 4096 x 11008 Q8_0 T = 384 231 / 134. Its error against 64 bits is below gemmh's on each (1.4e-7 against 2.4e-7
+// for the first). With its loads from memory left out it took 463 of 617 us, with its LDS reads left out too 414; at
+// full load the card runs it at 2.0 GHz.
+// Measured and not kept: the loads staged through registers (644 against 607 us), a ring of 4 one-block stages (623
+// against 617, 113 against 106), loads spread over the stage's arithmetic (738 against 735).
+template <int KIND, int NJ, int GR>
+__device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const uint8_t *__restrict__ img, float *__restrict__ y, u32 rows,
+                                           u32 nb, const float *__restrict__ bias, const float *__restrict__ res, u32 T, u32 ys, u32 rs,
+                                           float *__restrict__ part, u32 nfull, u32 nsplit) {
+  constexpr bool Q4K = KIND == AMDC_Q4_K, Q6 = KIND == AMDC_Q6_K, Q8 = KIND == AMDC_Q8_0, PB = Q8 || KIND == AMDC_Q4_0; // PB: a d per block
+  constexpr u32 TW = 64u * NJ, SB = gw_stage(Q4K, TW), NB = SB / 1024u; // a stage's image, in 1 KB loads
+  constexpr u32 NF = NB / 4u, NR = NB % 4u;                            // whole rounds of the group's 4 waves, and the rest
+  constexpr u32 NA = Q8 ? 8u : 4u, NX = Q6 ? 2u : 0u, OA = NB * 1024u, OX = OA + NA * 1024u, STAGE = OX + NX * 1024u;
+  // a ring of 2 stages (one in flight), or of 3 where 64 tokens leave the LDS and a stage is shorter than a load's
+  // way from memory (the 64-token tiles; one in flight is what fits beside the 128-token ones)
+  constexpr u32 NBUF = NJ == 1 ? 3u : 2u, NWAIT = (NBUF - 2u) * (NF + NA / 4u);
+  constexpr u32 TB = PB ? 4096u : 8704u, HS = Q6 ? 2048u : 1024u; // a super-group's tables; the headers of 64 rows
+  constexpr u32 OT = NBUF * STAGE, OH = OT + 2u * TB, GL = OH + 2u * HS; // a group's LDS: ring, two tables, headers
+  constexpr u32 OSTR = 132u;                                        // floats per token of the output tile in the LDS
+  constexpr u32 OB = TW * OSTR * 4u;
+  static_assert(NR >= 1u && NR <= 3u && !(Q6 && NR != 1u), "the last loads of a stage");
+  __shared__ __attribute__((aligned(1024))) uint8_t sm_[GR * GL > OB ? GR * GL : OB];
+  const u32 tid = threadIdx.x, lane = tid & 63u, w = __builtin_amdgcn_readfirstlane(tid >> 6) & (4u * GR - 1u);
+  const u32 grp = GR == 2 ? w >> 2 : 0u, wq = w & 3u, wm = w & 1u, wn = (w >> 1) & 1u, l32 = lane & 31u, kg = lane >> 5;
+  const u32 ng = amdc_ngroups(nb);
+  const u32 ntt = (T + TW - 1u) / TW, b = blockIdx.x, full = b < nfull;
+  const u32 tail = (rows + 127u) / 128u * ntt - nfull, tj = b - nfull;
+  // whole-K tiles: the token tiles of a row tile on one XCD, as in gemmh_body
+  const u32 xg = 8u * ntt, xd = b / xg, xj = b % xg;
+  const u32 tile = full ? (b < nfull / xg * xg ? (8u * xd + xj % 8u) * ntt + xj / 8u : b) : nfull + tj % tail;
+  const u32 tt = tile % ntt, rt = tile / ntt;
+  const u32 ks = full ? 0u : tj / tail, nks = full ? 1u : nsplit, g0 = ng * ks / nks, g1 = ng * (ks + 1u) / nks;
+  const u32 r0 = nfull / ntt * 128u;
+  const u32 RB = (u32)amdc_row_bytes_k(KIND, nb);
+  const __amdgpu_buffer_rsrc_t rw = rsrc(W + (u64)rt * 128u * RB, min(128u, rows - rt * 128u) * RB);
+  const __amdgpu_buffer_rsrc_t rx = rsrc(img + (u64)tt * 4u * ng * SB, 4u * ng * SB);
+  uint8_t *sm = sm_ + grp * GL;
+
+  // a group's 1 KB loads of a stage, in its LDS in this order: NB of the image, NA of the weights (a 16-byte
+  // plane of 64 rows each), Q6_K: 2 of the high bits. Wave wq issues every fourth, and at least NF + NA / 4
+  const u32 vb = 16u * lane, va = lane * RB;
+  auto put = [&](__amdgpu_buffer_rsrc_t r, uint8_t *d, u32 vo) { lds_load16(r, (__attribute__((address_space(3))) void *)d, vo); };
+  auto plane = [&](u32 g, u32 p) { // the byte of plane p (Q8_0: two per block) of super-group g in its row
+    return (u32)(Q8 ? amdc_q8_off(ng, g, p) : Q6 ? amdc_q6k_nib_off(ng, g, p) : amdc_nib_off(ng, g, p));
+  };
+  auto doff = [&](u32 g) { return (u32)amdc_q6k_d_off(ng, g) & ~15u; };
+  auto issue = [&](u32 g, u32 q, u32 slot) { // super-group g, sub-blocks 2q, 2q + 1
+    const u32 far = g < g1 ? 0u : 0x40000000u; // past the range: out of the resources, zeros
+    const u32 bo = (4u * g + q) * SB + far, ro = 64u * (wq & 1u) * RB + far;
+    uint8_t *base = sm + slot * STAGE;
+    if (wq < NR) {
+      put(rx, base + (4u * NF + wq) * 1024u, vb + bo + (4u * NF + wq) * 1024u);
+    } else if (Q6 && wq < 3u) {
+      put(rw, base + OX + (wq - 1u) * 1024u, va + 64u * (wq - 1u) * RB + (u32)amdc_q6k_hi_off(ng, g, q) + far);
+    }
+#pragma unroll
+    for (u32 n = 0; n < NF; n++) put(rx, base + (wq + 4u * n) * 1024u, vb + bo + (wq + 4u * n) * 1024u);
+#pragma unroll
+    for (u32 n = 0; n < NA / 4u; n++) put(rw, base + OA + (wq + 4u * n) * 1024u, va + ro + plane(g, NA / 2u * q + (wq >> 1) + 2u * n));
+  };
+  auto heads = [&](u32 g) { // the headers of super-group g (Q6_K: its scales, and the 16 bytes that hold its d), by waves 2 and 3
+    if (wq < 2u) return;
+    put(rw, sm + OH + (wq - 2u) * HS, va + 64u * (wq - 2u) * RB + 16u * g);
+    if (Q6) put(rw, sm + OH + (wq - 2u) * HS + 1024u, va + 64u * (wq - 2u) * RB + doff(g));
+  };
+  // the tables of 64 rows (rb ..) of super-group g from their headers: thread (row, blocks 2 wq, 2 wq + 1):
+  //   Q4_K: sc [block pair][row] x 2 blocks: f16 (sc, sc / 16); at 4096 min [2][row]: - dmin mn of the 8 blocks as
+  //         two bf16 parts (at most 17 bits: the part rounded to nearest leaves at most 8); at 8192 d [row] f32
+  //   Q6_K: sc [block pair][row] x 2 blocks x 2 halves: f16 (sc >> 4, (sc & 15) / 16); at 8192 16 d [row] f32
+  //   Q4_0, Q8_0: d [block][row] f32
+  auto build = [&](u32 g, u32 rb, u32 par) {
+    uint8_t *t = sm + OT + par * TB;
+    const uint8_t *hc = sm + OH + rb / 64u * HS;
+    const u32x4 h = *(const u32x4 *)(hc + 16u * lane);
+    const u32 r = rb + lane;
+    if constexpr (PB) {
+      const u32 d2 = hword(h, wq);
+      float *o = (float *)t + 256u * wq + r;
+      o[0] = h2f(d2), o[128] = h2f(d2 >> 16);
+    } else if constexpr (Q6) {
+      const u32 sc = hword(h, wq);
+      u32x4 o;
+#pragma unroll
+      for (u32 e = 0; e < 4u; e++) {
+        const _Float16 f = (_Float16)(short)((int)(sc << (24u - 8u * e)) >> 28), l = (_Float16)(unsigned short)((sc >> (8u * e)) & 15u) * (_Float16)0.0625f;
+        o[e] = (u32)__builtin_bit_cast(unsigned short, f) | ((u32)__builtin_bit_cast(unsigned short, l) << 16);
+      }
+      *(u32x4 *)(t + (wq * 128u + r) * 16u) = o;
+      if (wq == 0u) *(float *)(t + 8192u + r * 4u) = 16.0f * h2f(*(const unsigned short *)(hc + 1024u + 16u * lane + 2u * (g & 7u)));
+    } else {
+      const u32 s2 = (u32)((((u64)h.z << 32) | h.y) >> (12u * wq)), n2 = (u32)((((u64)h.w << 32) | h.z) >> (16u + 12u * wq));
+      const h2 sc = __builtin_bit_cast(h2, (s2 & 63u) | ((s2 & 0xFC0u) << 10) | 0x64006400u) - (h2){(_Float16)1024.0f, (_Float16)1024.0f};
+      const h2 sd = sc * (h2){(_Float16)0.0625f, (_Float16)0.0625f};
+      const u32 a = __builtin_bit_cast(u32, sc), c = __builtin_bit_cast(u32, sd);
+      *(u32x2 *)(t + (wq * 128u + r) * 8u) = (u32x2){__builtin_amdgcn_perm(c, a, 0x05040100u), __builtin_amdgcn_perm(c, a, 0x07060302u)};
+      const float dm = -h2f(h.x >> 16), m0 = dm * (float)(n2 & 63u), m1 = dm * (float)((n2 >> 6) & 63u);
+      const u32 p0 = __builtin_bit_cast(u32, m0) + 0x8000u, p1 = __builtin_bit_cast(u32, m1) + 0x8000u;
+      const float q0 = m0 - __builtin_bit_cast(float, p0 & 0xFFFF0000u), q1 = m1 - __builtin_bit_cast(float, p1 & 0xFFFF0000u);
+      u32 *l = (u32 *)(t + 4096u + r * 16u + 4u * wq);
+      l[0] = __builtin_amdgcn_perm(p1, p0, 0x07060302u);
+      l[512] = __builtin_amdgcn_perm(__builtin_bit_cast(u32, q1), __builtin_bit_cast(u32, q0), 0x07060302u);
+      if (wq == 0u) *(float *)(t + 8192u + r * 4u) = h2f(h.x);
+    }
+  };
+
+  v16f acc[2][NJ], tmp[PB ? 1 : 2][NJ];
+#pragma unroll
+  for (u32 i = 0; i < 2u; i++)
+#pragma unroll
+    for (u32 j = 0; j < (u32)NJ; j++) acc[i][j] = (v16f)(0.0f), tmp[PB ? 0u : i][j] = (v16f)(0.0f);
+  const KW kc = kw();
+  // the first super-group's headers and tables
+  u32 g = g0 + grp, par = 0u, slot = 0u;
+  heads(g);
+  issue(g, 0u, 0u);
+  if (NBUF == 3u) issue(g, 1u, 1u);
+  vm_wait(0u);
+  v8_barrier();
+  build(g, 0u, 0u);
+  build(g, 64u, 0u);
+  if (GR == 2 && grp) __builtin_amdgcn_s_barrier(); // the second group runs half a stage behind the first
+  // lane offsets inside a stage
+  const u32 rl = 64u * wm + l32;
+  const u32 la = OA + rl * 16u + (Q8 ? 2048u * kg : 8u * kg), lb = 2u * NJ * wn * 1024u + 16u * lane, ld = 128u * TW + 4u * (32u * NJ * wn + l32);
+  const u32 lx = 128u * TW + 1024u + (NJ == 2 ? 1024u * wn : 0u) + 16u * lane;
+  // the A operands of block bb of stage q, row tile i (Q6_K: [s] hi, [2 + s] lo)
+  constexpr u32 NFR = Q6 ? 4u : 2u;
+  auto frag = [&](const uint8_t *base, const uint8_t *tb, u32 q, u32 bb, u32 i, h8 *af) {
+    if constexpr (Q8) {
+      const u32x4 wv = *(const u32x4 *)(base + la + 4096u * bb + 512u * i);
+      af[0] = a_frag_q8(wv.x, wv.y), af[1] = a_frag_q8(wv.z, wv.w);
+    } else if constexpr (Q6) {
+      const u32x2 sp = *(const u32x2 *)(tb + (q * 128u + rl + 32u * i) * 16u + 8u * bb);
+      const u32x2 wv = *(const u32x2 *)(base + la + 2048u * bb + 512u * i), hw = *(const u32x2 *)(base + OX + (rl + 32u * i) * 16u + 8u * bb);
+#pragma unroll
+      for (u32 s = 0; s < 2u; s++) {
+        const u32 t = (s ? hw.y : hw.x) >> (4u * kg);
+        const u32 q0 = ((wv.x >> (4u * s)) & 0x0F0F0F0Fu) | ((t << 4) & 0x30303030u), q1 = ((wv.y >> (4u * s)) & 0x0F0F0F0Fu) | ((t << 2) & 0x30303030u);
+        a_frag_w6(q0, q1, __builtin_bit_cast(h2, s ? sp.y : sp.x), af[s], af[2u + s]);
+      }
+    } else {
+      const u32x2 wv = *(const u32x2 *)(base + la + 2048u * bb + 512u * i);
+      h2 s = {(_Float16)1.0f, (_Float16)0.0625f}, c = {(_Float16)-1032.0f, (_Float16)-72.0f};
+      if constexpr (Q4K) {
+        s = __builtin_bit_cast(h2, *(const u32 *)(tb + (q * 128u + rl + 32u * i) * 8u + 4u * bb));
+        c = s * (h2){(_Float16)-1024.0f, (_Float16)-1024.0f};
+      }
+      af[0] = a_frag_w(wv.x, s, c, kc), af[1] = a_frag_w(wv.y, s, c, kc);
+    }
+  };
+  auto mma = [&](const h8 *af, const h8 *bf) {
+    v16f x = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[0], bf[0], (v16f)(0.0f), 0, 0, 0);
+    x = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[1], bf[1], x, 0, 0, 0);
+    if constexpr (Q6) {
+      x = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[2], bf[0], x, 0, 0, 0);
+      x = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[3], bf[1], x, 0, 0, 0);
+    }
+    return x;
+  };
+  const u32 nit = (g1 - g0 + GR - 1u) / GR;
+  for (u32 it = 0; it < nit; it++, g += GR, par ^= 1u) {
+    const uint8_t *tb = sm + OT + par * TB;
+    const bool on = g < g1; // (the last super-group of an odd range is the first group's)
+#pragma unroll
+    for (u32 q = 0; q < 4u; q++) {
+      vm_wait(NWAIT); // this stage's loads have landed ...
+      v8_barrier();   // ... in every wave of the group, and every wave is done with the stage before
+      const u32 sl = NBUF == 2u ? q & 1u : slot, nsl = NBUF == 2u ? sl ^ 1u : sl ? sl - 1u : 2u; // the slot of the stage before
+      if (NBUF == 3u) slot = sl == 2u ? 0u : sl + 1u;
+      if (q == 0u) heads(g + GR);
+      issue(q + NBUF - 1u < 4u ? g : g + GR, (q + NBUF - 1u) & 3u, nsl);
+      const uint8_t *base = sm + sl * STAGE;
+#pragma unroll
+      for (u32 bb = 0; bb < 2u; bb++) {
+        if (GR == 2 && bb == 1u) __builtin_amdgcn_s_barrier(); // the other group's stage begins
+        __builtin_amdgcn_sched_barrier(0);
+        if (!on) continue;
+        h8 bf[NJ][2], af[Q6 ? 1 : 2][NFR]; // Q6_K: one row tile's operands at a time (registers)
+#pragma unroll
+        for (u32 i = 0; i < (Q6 ? 1u : 2u); i++) frag(base, tb, q, bb, i, af[i]);
+#pragma unroll
+        for (u32 j = 0; j < (u32)NJ; j++)
+#pragma unroll
+          for (u32 s = 0; s < 2u; s++) bf[j][s] = *(const h8 *)(base + lb + 64u * TW * bb + (2u * j + s) * 1024u);
+        if constexpr (PB) {
+          // d_w d_a of the tile's rows and tokens as an outer product on the matrix unit (rank 1, one rounding), row tiles 0
+          // and 1 in its two blocks; then acc += (d_w d_a) X per element
+          const float dw = *(const float *)(tb + ((2u * q + bb) * 128u + rl + 32u * kg) * 4u);
+          v32f pr[NJ];
+#pragma unroll
+          for (u32 j = 0; j < (u32)NJ; j++) {
+            const float dj = *(const float *)(base + ld + 4u * TW * bb + 128u * j);
+            pr[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dj, (v32f)(0.0f), 0, 0, 0);
+          }
+          v16f x[2];
+          x[0] = mma(af[0], bf[0]);
+#pragma unroll
+          for (u32 t = 0; t < 2u * NJ; t++) {
+            if (t + 1u < 2u * NJ) x[(t + 1u) & 1u] = mma(af[(t + 1u) / NJ], bf[(t + 1u) % NJ]);
+            const u32 i = t / NJ, j = t % NJ;
+#pragma unroll
+            for (u32 v = 0; v < 16u; v++) acc[i][j][v] = __builtin_fmaf(pr[j][16u * i + v], x[t & 1u][v], acc[i][j][v]);
+          }
+        } else {
+          float dj[NJ];
+#pragma unroll
+          for (u32 j = 0; j < (u32)NJ; j++) dj[j] = *(const float *)(base + ld + 4u * TW * bb + 128u * j);
+          v16f x[2];
+          x[0] = mma(af[0], bf[0]);
+#pragma unroll
+          for (u32 t = 0; t < 2u * NJ; t++) {
+            if (Q6 && t + 1u == (u32)NJ) {
+              __builtin_amdgcn_sched_barrier(0);
+              frag(base, tb, q, bb, 1u, af[0]);
+            }
+            if (t + 1u < 2u * NJ) x[(t + 1u) & 1u] = mma(af[Q6 ? 0u : (t + 1u) / NJ], bf[(t + 1u) % NJ]);
+            const u32 i = t / NJ, j = t % NJ;
+#pragma unroll
+            for (u32 v = 0; v < 16u; v++)
+              tmp[i][j][v] = q == 0u && bb == 0u ? dj[j] * x[t & 1u][v] : __builtin_fmaf(dj[j], x[t & 1u][v], tmp[i][j][v]);
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (!PB && on) {
+        // Q4_K: the min term of one of the wave's token groups: - (dmin mn) (d_a asum) over the super-group's 8 blocks,
+        // m1 x1 + m1 x2 + m2 x1 + m2 x2 + m1 x3 + m2 x3
+        if (Q4K && (NJ == 2 || wn == (q >> 1))) {
+          const u32 j = NJ == 2 ? q >> 1 : 0u;
+          const b8 xb = *(const b8 *)(base + lx);
+#pragma unroll
+          for (u32 i = 0; i < 2u; i++) {
+            const uint8_t *l = tb + 4096u + (rl + 32u * i) * 16u;
+            if ((q & 1u) == 0u) {
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const b8 *)l, xb, acc[i][j], 0, 0, 0);
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const b8 *)(l + 2048u), xb, acc[i][j], 0, 0, 0);
+            } else {
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const b8 *)(l + 2048u * kg), xb, acc[i][j], 0, 0, 0);
+            }
+          }
+        }
+        if (q == 3u) { // the end of the super-block: d of the C rows 8 (v / 4) + 4 kg + v % 4
+#pragma unroll
+          for (u32 i = 0; i < 2u; i++)
+#pragma unroll
+            for (u32 v4 = 0; v4 < 4u; v4++) {
+              const v4f dv = *(const v4f *)(tb + 8192u + (64u * wm + 32u * i + 8u * v4 + 4u * kg) * 4u);
+#pragma unroll
+              for (u32 v = 0; v < 4u; v++)
+#pragma unroll
+                for (u32 j = 0; j < (u32)NJ; j++)
+                  acc[i][j][4u * v4 + v] = __builtin_fmaf(dv[v], tmp[PB ? 0u : i][j][4u * v4 + v], acc[i][j][4u * v4 + v]);
+            }
+        }
+      }
+      // the next super-group's headers, loaded in stage 0 ahead of stage NBUF - 1, have landed by stage NBUF - 1
+      if (q == NBUF - 1u) build(g + GR, 0u, par ^ 1u);
+      if (q == 3u) build(g + GR, 64u, par ^ 1u);
+    }
+  }
+  if (GR == 2 && !grp) __builtin_amdgcn_s_barrier();
+  // the groups' sums through the LDS ([token][row]), then the tile's rows in order
+  vm_wait(0u);
+  v8_barrier();
+  float *so = (float *)sm_;
+#pragma unroll
+  for (u32 ph = 0; ph < (u32)GR; ph++) {
+    if (GR == 1 || grp != ph) {
+#pragma unroll
+      for (u32 i = 0; i < 2u; i++)
+#pragma unroll
+        for (u32 j = 0; j < (u32)NJ; j++)
+#pragma unroll
+          for (u32 v4 = 0; v4 < 4u; v4++) {
+            v4f *o = (v4f *)&so[(32u * (NJ * wn + j) + l32) * OSTR + 64u * wm + 32u * i + 8u * v4 + 4u * kg];
+            v4f a = {acc[i][j][4u * v4], acc[i][j][4u * v4 + 1u], acc[i][j][4u * v4 + 2u], acc[i][j][4u * v4 + 3u]};
+            if (ph == 1u) a = a + *o;
+            *o = a;
+          }
+    }
+    v8_barrier();
+  }
+  const u32 ro = tid & 127u, r = rt * 128u + ro;
+  if (r < rows) {
+    const float bv = full && bias ? bias[r] : 0.0f;
+#pragma unroll 4
+    for (u32 t = tid >> 7; t < TW; t += 2u * GR) {
+      const u32 tk = tt * TW + t;
+      if (tk >= T) break;
+      float o = so[t * OSTR + ro];
+      if (!full) {
+        part[((u64)ks * T + tk) * (rows - r0) + (r - r0)] = o;
+      } else {
+        if (bias) o = o + bv;
+        if (res) o = res[(u64)tk * rs + r] + o;
+        y[(u64)tk * ys + r] = o;
+      }
+    }
+  }
+}
+#define GEMMW_KERNEL(KN, NJ, KIND, GR)                                                                                              \
+  extern "C" __global__ __launch_bounds__(256 * GR, 2) void amdc_gemmw_##KN(const uint8_t *W, const uint8_t *img, float *y, u32 rows, u32 nb, \
+                                                                    const float *bias, const float *res, u32 T, u32 ys, u32 rs,  \
+                                                                    float *part, u32 nfull, u32 nsplit) {                        \
+    gemmw_body<KIND, NJ, GR>(W, img, y, rows, nb, bias, res, T, ys, rs, part, nfull, nsplit);                                    \
+  }
+// per kind: 128 and 64 tokens in two groups, 128 tokens in one
+#define GEMMW_KERNELS(KN, KIND)      \
+  GEMMW_KERNEL(KN##_n128, 2, KIND, 2) \
+  GEMMW_KERNEL(KN##_n64, 1, KIND, 2)
+GEMMW_KERNELS(q4_0, AMDC_Q4_0)
+GEMMW_KERNELS(q4_k, AMDC_Q4_K)
+GEMMW_KERNELS(q6_k, AMDC_Q6_K)
+GEMMW_KERNELS(q8_0, AMDC_Q8_0)
+GEMMW_KERNEL(q4_0_i128, 2, AMDC_Q4_0, 1)
+GEMMW_KERNEL(q4_k_i128, 2, AMDC_Q4_K, 1)
+GEMMW_KERNEL(q6_k_i128, 2, AMDC_Q6_K, 1)
 
 template <int KIND, int NS, int NH, int WS>
 __device__ __forceinline__ void gemv8_body(const uint8_t *__restrict__ W, const uint8_t *__restrict__ xq, float *__restrict__ y, u32 rows,

@@ -214,8 +214,8 @@ int amdc_gemv_q6k_t(const void *w, const uint8_t *xq, float *y, uint32_t rows, u
  * ie_gemm_q4kr (kernels/ie_kernels.c:1289, src/hip.c:998-1001). The integer
  * sums of the sub-blocks are exact: by default on the f16 MFMA with the 6-bit
  * scale folded into the weights (q sc <= 945 and the int8 activations are f16
- * integers; every partial sum is an integer below 2^24), or on the int8 MFMA
- * (tuning); f32 outputs within 1e-5 of cpu_gemv_q4k per token row. Uses a
+ * integers; every partial sum is an integer below 2^24; the min term on the bf16
+ * MFMA from exact parts), or on the int8 MFMA (tuning); f32 outputs within 1e-5 of cpu_gemv_q4k per token row. Uses a
  * device workspace that the library allocates on the first call of a size
  * (call once outside graph capture before capturing). */
 int amdc_gemm_q4k(const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res,
@@ -252,7 +252,8 @@ int amdc_op_gemv(int kind, const void *w, const uint8_t *xq, float *y, uint32_t 
 /* amdc_op_gemv without any device allocation, for callers that cannot allocate (code under
  * HIP graph capture on a workspace size not seen before, tight serving loops, hosts that
  * forbid hipMalloc). No reference counterpart. The same kernels and launch choices as
- * amdc_op_gemv, so the same bits; the workspace (split-K partial sums, the GEMM's prepared
+ * amdc_op_gemv, so the same bits (a GEMM whose default kernels' workspace does not fit runs on
+ * kernels and splits that need less, within the same bounds); the workspace (split-K partial sums, the GEMM's prepared
  * activations) is a fixed device array of AMDC_SCRATCH_BYTES in the code object, held by the
  * device from amdc_open until amdc_close. A call whose workspace would exceed it fails with
  * AMDC_EINVAL before any launch (e.g. T = 256 prefill chunks fit up to about 17408 x 5120
@@ -274,7 +275,7 @@ int amdc_block_dots(int kind, const void *w, const uint8_t *xq, int32_t *out, ui
  * two); the decode kernel (0: the pipelined one; 1 or 2: the multi-vector
  * kernel with 1 or 2 super-groups of loads per step); workgroups of a GEMV
  * launch; the GEMM kernel (1, 2: int8 MFMA with 64 or 128 tokens per
- * workgroup; 3, 4, 5: f16 MFMA, rows x tokens 64x128, 64x64, 128x128 (Q4_K));
+ * workgroup; 3, 4: f16 MFMA, rows x tokens 64x128, 64x64; 5: the wide f16-MFMA tiles at any size);
  * the GEMM's K split (1..16); the decode kernel's form when gemv_unroll is 0
  * (1: the persistent pipelined form, 2: the buffer-load form that keeps the
  * next super-group in flight, 3: the single-shot form, one row group per
