@@ -284,8 +284,12 @@ enum {
   K_GEMVS1W = K_GEMVM8 + 2,     /* amdc_gemv_q4_0_s1w, amdc_gemv_q4_k_s1w */
   K_GEMMW_PREP = K_GEMVS1W + 2,
   K_GEMMW, /* amdc_gemmw_q4_0_n128, _n64, _i128, the same of q4_k and q6_k, amdc_gemmw_q8_0_n128, _n64 */
-  K_N = K_GEMMW + 11
+  K_QUANT_V = K_GEMMW + 11, /* the producers on aligned rows: amdc_quant_q8_v, amdc_swiglu_q8_v, amdc_rmsnorm_q8_r */
+  K_SWIGLU_V,
+  K_RMSNORM_R,
+  K_N
 };
+#define KN(s) "amdc_" s
 #define GW(s) "amdc_gemmw_" s
 static const char *const kname[K_N] = {
     "amdc_quant_q8",           "amdc_dots_q4_0",          "amdc_dots_q4_k",          "amdc_gemm_q4_k_n128",
@@ -310,7 +314,8 @@ static const char *const kname[K_N] = {
     "amdc_gemv_q8_0_pn",       "amdc_gemv_q6_k_pn",
     "amdc_gemv_q8_0_m1",       "amdc_gemv_q6_k_m1",       "amdc_gemv_q4_0_s1w",      "amdc_gemv_q4_k_s1w",
     GW("prep"), GW("q4_0_n128"), GW("q4_0_n64"), GW("q4_0_i128"), GW("q4_k_n128"), GW("q4_k_n64"), GW("q4_k_i128"),
-    GW("q6_k_n128"), GW("q6_k_n64"), GW("q6_k_i128"), GW("q8_0_n128"), GW("q8_0_n64")};
+    GW("q6_k_n128"), GW("q6_k_n64"), GW("q6_k_i128"), GW("q8_0_n128"), GW("q8_0_n64"),
+    KN("quant_q8_v"), KN("swiglu_q8_v"), KN("rmsnorm_q8_r")};
 
 static hipModule_t g_mod;
 static hipFunction_t g_k[K_N];
@@ -651,6 +656,8 @@ static int launch(int k, unsigned gx, unsigned gy, unsigned lds, void *stream, v
 const char *amdc_last_kernel(void) { return g_last_k >= 0 ? kname[g_last_k] : ""; }
 
 static int aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
+/* every row of an array of rows at a stride of s bytes lies on a multiple of al bytes */
+static int vec_rows(const void *p, uint32_t s, uint32_t al) { return (((uintptr_t)p | s) & (al - 1u)) == 0; }
 
 int amdc_quant_q8(const float *x, uint8_t *q, uint32_t nb, uint32_t T, uint32_t xs, uint32_t qs, void *stream) {
   NEED_OPEN();
@@ -663,6 +670,7 @@ int amdc_quant_q8(const float *x, uint8_t *q, uint32_t nb, uint32_t T, uint32_t 
     return rec_put(&o);
   }
   void *args[] = {&x, &q, &nb, &xs, &qs};
+  if (vec_rows(x, T > 1u ? xs : 0u, 16u) && vec_rows(q, T > 1u ? qs : 0u, 4u)) return launch(K_QUANT_V, (nb + 31u) / 32u, T, 0, stream, args);
   return launch(K_QUANT, (nb + 7u) / 8u, T, 0, stream, args);
 }
 
@@ -679,6 +687,11 @@ int amdc_rmsnorm_q8(const float *x, const float *w, float *y, uint32_t n, float 
     return rec_put(&o);
   }
   void *args[] = {&x, &w, &y, &n, &eps, &q, &xs, &ys, &qs};
+  /* a workgroup per row from 96 rows (fewer leave most CUs idle), 2^19 values and rows of 1024 (shorter ones
+     leave lanes idle): amdc_rmsnorm_q8_r lists the measurements */
+  if (T >= 96u && n >= 1024u && (u64)T * n >= (1u << 19) && aligned16(w) && vec_rows(x, T > 1u ? xs : 0u, 16u) && vec_rows(y, T > 1u ? ys : 0u, 16u) &&
+      vec_rows(q, T > 1u && q ? qs : 0u, 4u))
+    return launch(K_RMSNORM_R, 1, T, 0, stream, args);
   return launch(K_RMSNORM_Q8, (n / 32u + 7u) / 8u, T, 0, stream, args);
 }
 
@@ -694,6 +707,8 @@ int amdc_swiglu_q8(float *a, const float *b, uint32_t n, uint8_t *q, uint32_t T,
     return rec_put(&o);
   }
   void *args[] = {&a, &b, &n, &q, &as, &qs};
+  if (aligned16(b) && vec_rows(a, T > 1u ? as : 0u, 16u) && vec_rows(q, T > 1u && q ? qs : 0u, 4u))
+    return launch(K_SWIGLU_V, (n + 1023u) / 1024u, T, 0, stream, args);
   return launch(K_SWIGLU_Q8, (n + 255u) / 256u, T, 0, stream, args);
 }
 

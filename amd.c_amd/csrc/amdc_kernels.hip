@@ -207,6 +207,37 @@ extern "C" __global__ __launch_bounds__(256) void amdc_quant_q8(const float *__r
   }
 }
 
+// The Q8 copy of 4 consecutive values per lane, 8 lanes per block of 32: the same d, q and asum as above (max and
+// integer sums are exact in any order), one 32-bit store of q per lane. on: uniform over the 8 lanes.
+__device__ __forceinline__ void quant_vec4(const v4f &x, u32 b, bool on, uint8_t *__restrict__ q, u32 nb) {
+  const u32 e = threadIdx.x & 7u;
+  float a = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(x.x), __builtin_fabsf(x.y)), __builtin_fmaxf(__builtin_fabsf(x.z), __builtin_fabsf(x.w)));
+  a = __builtin_fmaxf(a, dpp<0xB1>(a));
+  a = __builtin_fmaxf(a, dpp<0x4E>(a));
+  a = __builtin_fmaxf(a, dpp<0x141>(a));
+  const float d = a / 127.0f;
+  int qi[4];
+  q8_round4(x, d, qi);
+  u32 sum = (u32)qi[0] + (u32)qi[1] + (u32)qi[2] + (u32)qi[3];
+  sum += (u32)__builtin_amdgcn_update_dpp(0, (int)sum, 0xB1, 0xF, 0xF, false);
+  sum += (u32)__builtin_amdgcn_update_dpp(0, (int)sum, 0x4E, 0xF, 0xF, false);
+  sum += (u32)__builtin_amdgcn_update_dpp(0, (int)sum, 0x141, 0xF, 0xF, false);
+  if (!on) return;
+  ((u32 *)(q + 32u * b))[e] = (u32)(qi[0] & 255) | (u32)(qi[1] & 255) << 8 | (u32)(qi[2] & 255) << 16 | (u32)qi[3] << 24;
+  if (e == 0u) ((float *)(q + 32u * nb))[b] = d, ((u32 *)(q + 36u * nb))[b] = sum;
+}
+
+// amdc_quant_q8 on 16-byte aligned rows of x and 4-byte aligned rows of q: 128-bit loads, a quarter of the
+// instructions per value, which bound it. Grid (ceil(nb / 32), T). Measured on MI355X (us): nb = 160,
+// T = 1024 13.3 / 6.7, T = 256 4.6 / 3.1, T = 8 2.2 / 2.2 (the form above / this)
+extern "C" __global__ __launch_bounds__(256) void amdc_quant_q8_v(const float *__restrict__ x, uint8_t *__restrict__ q, u32 nb, u32 xs, u32 qs) {
+  x = (const float *)((const uint8_t *)x + (u64)blockIdx.y * xs);
+  q += (u64)blockIdx.y * qs;
+  const u32 b = blockIdx.x * 32u + (threadIdx.x >> 3);
+  const bool on = b < nb;
+  quant_vec4(*(const v4f *)(x + 32u * (on ? b : nb - 1u) + 4u * (threadIdx.x & 7u)), b, on, q, nb);
+}
+
 // The Q8 producers of a decode step, fused as the reference fuses them
 // (kernels/ie_kernels.c:240-265 ie_rmsnorm, :2458 ie_swiglu): the float result
 // and its Q8 copy (the arithmetic of amdc_quant_q8 on that result) in one
@@ -378,6 +409,45 @@ extern "C" __global__ __launch_bounds__(256) void amdc_swiglu_q8(float *__restri
   const float v = swiglu1(a[i], b[i]);
   a[i] = v;
   if (q) quant_half(v, i >> 5, q, n >> 5);
+}
+
+// The same on 16-byte aligned rows of a and b and 4-byte aligned rows of q: 4 values per lane. Grid (ceil(n / 1024),
+// T). Measured on MI355X (us): n = 17408, T = 256 14.6 / 8.6, T = 8 2.4 / 2.3 (the form above / this)
+extern "C" __global__ __launch_bounds__(256) void amdc_swiglu_q8_v(float *__restrict__ a, const float *__restrict__ b, u32 n, uint8_t *__restrict__ q,
+                                                                  u32 as, u32 qs) {
+  a = (float *)((uint8_t *)a + (u64)blockIdx.y * as);
+  b = (const float *)((const uint8_t *)b + (u64)blockIdx.y * as);
+  const u32 i = 4u * (blockIdx.x * NT + threadIdx.x);
+  const bool on = i < n; // whole blocks of 32 (8 lanes) at once
+  const u32 j = on ? i : n - 4u;
+  const v4f g = *(const v4f *)(a + j), u = *(const v4f *)(b + j);
+  v4f v;
+#pragma unroll
+  for (u32 m = 0; m < 4u; m++) v[m] = swiglu1(g[m], u[m]);
+  if (on) *(v4f *)(a + i) = v;
+  if (q) quant_vec4(v, i >> 5, on, q + (u64)blockIdx.y * qs, n >> 5);
+}
+
+// amdc_rmsnorm_q8 with a workgroup per row, for many rows: the other form's n / 256 workgroups per row each read it
+// all for the sum of squares (the same code here, so the same s); then 4 values per lane, the row again from L1 / L2.
+// 16-byte aligned rows of x, y and w, 4-byte aligned rows of q. Grid (1, T). Measured on MI355X (us): n = 5120, T = 256 13.6 / 6.2,
+// T = 512 22.6 / 7.4, T = 64 4.4 / 5.4; n = 5376, T = 98 6.6 / 6.2; n = 4096, T = 128 4.8 / 4.6; n = 1024, T = 512
+// 4.7 / 3.6; 256, 2048 4.0 / 4.7; 8192, 64 6.0 / 7.0; 17408, 32 10.1 / 12.6 (the other form / this)
+extern "C" __global__ __launch_bounds__(256) void amdc_rmsnorm_q8_r(const float *__restrict__ x, const float *__restrict__ w, float *__restrict__ y,
+                                                                   u32 n, float eps, uint8_t *__restrict__ q, u32 xs, u32 ys, u32 qs) {
+  __shared__ float s_ss[4];
+  x = (const float *)((const uint8_t *)x + (u64)blockIdx.y * xs);
+  y = (float *)((uint8_t *)y + (u64)blockIdx.y * ys);
+  if (q) q += (u64)blockIdx.y * qs;
+  const float s = rms_scale<false, 8u>(x, n, eps, s_ss);
+  for (u32 i0 = 0; i0 < n; i0 += 4u * NT) {
+    const u32 i = i0 + 4u * threadIdx.x;
+    const bool on = i < n; // whole blocks of 32 (8 lanes) at once
+    const v4f a = *(const v4f *)(x + (on ? i : 0u)), g = *(const v4f *)(w + (on ? i : 0u));
+    const v4f v = {a.x * s * g.x, a.y * s * g.y, a.z * s * g.z, a.w * s * g.w};
+    if (on) *(v4f *)(y + i) = v;
+    if (q) quant_vec4(v, i >> 5, on, q, n >> 5);
+  }
 }
 
 // ------------------------------------------------------------------ GEMV
