@@ -287,7 +287,8 @@ enum {
   K_QUANT_V = K_GEMMW + 11, /* the producers on aligned rows: amdc_quant_q8_v, amdc_swiglu_q8_v, amdc_rmsnorm_q8_r */
   K_SWIGLU_V,
   K_RMSNORM_R,
-  K_N
+  K_GEMVS8, /* amdc_gemv_q8_0_s1, _s2, _xs1, _xs2, amdc_gemv_q6_k_s1, (none), _xs1 */
+  K_N = K_GEMVS8 + 7
 };
 #define KN(s) "amdc_" s
 #define GW(s) "amdc_gemmw_" s
@@ -315,7 +316,8 @@ static const char *const kname[K_N] = {
     "amdc_gemv_q8_0_m1",       "amdc_gemv_q6_k_m1",       "amdc_gemv_q4_0_s1w",      "amdc_gemv_q4_k_s1w",
     GW("prep"), GW("q4_0_n128"), GW("q4_0_n64"), GW("q4_0_i128"), GW("q4_k_n128"), GW("q4_k_n64"), GW("q4_k_i128"),
     GW("q6_k_n128"), GW("q6_k_n64"), GW("q6_k_i128"), GW("q8_0_n128"), GW("q8_0_n64"),
-    KN("quant_q8_v"), KN("swiglu_q8_v"), KN("rmsnorm_q8_r")};
+    KN("quant_q8_v"), KN("swiglu_q8_v"), KN("rmsnorm_q8_r"),
+    KN("gemv_q8_0_s1"), KN("gemv_q8_0_s2"), KN("gemv_q8_0_xs1"), KN("gemv_q8_0_xs2"), KN("gemv_q6_k_s1"), KN("gemv_q6_k_s1"), KN("gemv_q6_k_xs1")};
 
 static hipModule_t g_mod;
 static hipFunction_t g_k[K_N];
@@ -922,9 +924,40 @@ static int gemvk_launch(int kind, const void *w, const void *in, int fq, float *
   return launch(k, nrg, S, 320u * R, stream, a);
 }
 
+/* The single-shot decode GEMV of the Q8_0 and Q6_K kinds (amdc_gemv_q8_0_s1 / _s2, amdc_gemv_q6_k_s1; with fq on an f32
+ * vector, _xs*, quantized in every workgroup): one super-group per lane; Q8_0 also two, for rows of more than 64, and
+ * with fq, as the Q4 kinds, while the grid is over 3 workgroups per CU and 8 lanes remain (22016 x 4096 16.2 us against
+ * 17.8; at 4 lanes 32000 x 2048 21.2 against 12.7). -1, nothing launched, where it is not the faster form
+ * (amdc_kernels.hip lists both sides): Q6_K rows of more than 64 super-groups, or on 2^16 rows and more a row that
+ * leaves a quarter of its lanes idle (100000 x 5120, 20 of 32 lanes, 77.1 us against 74.6; 100000 x 4096 54.9 against
+ * 58.0); Q8_0 rows of more than 128; with fq, where the workgroups quantize more than 2^17 blocks between them (us,
+ * fused / quantize launch and this form: 32000 x 4096 Q8_0 21.7 / 23.7, 32000 x 2048 Q6_K 12.3 / 14.2, 2048 x 5632 6.4 /
+ * 6.9; 20000 x 5120 Q6_K 24.9 / 20.0, 60000 x 3072 33.3 / 31.1, 4096 x 11008 17.8 / 12.1); and under the tuning knobs of
+ * the other forms. */
+static int gemvs8_launch(int kind, const void *w, const void *in, int fq, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res,
+                         uint8_t *q8, void *stream) {
+  const u32 ng = amdc_ngroups(nb), cus = g_cus > 0 ? (u32)g_cus : 256u;
+  const u64 rb = amdc_row_bytes_k(kind, nb);
+  if (t_lanes > 0 || t_wgs > 0 || (t_form != 0 && t_form != 3) || (u64)rows * rb + rb >= (1ull << 32)) return -1;
+  u32 L = 4u;
+  while (L < 64u && L < ng) L <<= 1;
+  if (kind == AMDC_KIND_Q6_K ? ng > 64u || (rows >= (1u << 16) && 4u * ng <= 3u * L) : ng > 128u) return -1;
+  if (fq && kind == AMDC_KIND_Q8_0 && L >= 16u && L >= ng && (rows + 4u * (64u / L) - 1u) / (4u * (64u / L)) > 3u * cus) L >>= 1;
+  const u32 ni = (ng + L - 1u) / L, rpg = 4u * (64u / L), nrg = (rows + rpg - 1u) / rpg;
+  if (fq && (u64)nrg * nb > (1u << 17)) return -1;
+  const int k = K_GEMVS8 + (kind == AMDC_KIND_Q6_K ? 4 : 0) + (fq ? 2 : 0) + (int)ni - 1;
+  const u32 lds = (kind == AMDC_KIND_Q6_K ? 352u : 320u) * ng;
+  void *a[] = {&w, &in, &y, &rows, &nb, &bias, &res, (void *)&L, &q8};
+  return launch(k, nrg, 1, lds, stream, a);
+}
+
 static int gemv_launch(int kind, const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias,
                        const float *res, uint32_t T, uint32_t xs, uint32_t ys, uint32_t rs, void *stream) {
   if (kind == AMDC_KIND_Q8_0 || kind == AMDC_KIND_Q6_K) {
+    if (T == 1u && t_unroll <= 0) {
+      const int rc = gemvs8_launch(kind, w, xq, 0, y, rows, nb, bias, res, NULL, stream);
+      if (rc != -1) return rc;
+    }
     if (T == 1u || t_unroll > 0) return gemv_k8_launch(kind, w, xq, y, rows, nb, bias, res, T, xs, ys, rs, stream);
     if (T <= 8u && t_ksplit == 0) {
       /* a few vectors on a small matrix: the decode items and arithmetic for every vector
@@ -1074,6 +1107,9 @@ static int gemvxw_pick(int kind, u32 ng, u32 rows, u32 *L, u32 *ni, u32 *nth) {
   return 0;
 }
 
+/* Q8_0 / Q6_K: the longest rows quantized inside the GEMV (MI355X, us, fused / quantize launch and GEMV: 2048 x 5632
+ * Q8_0 6.25 / 6.65, 4096 x 11008 17.7 / 13.4) */
+#define X8_FUSE_NB 192u
 static int gemv_x(int kind, const char *op, const void *w, const float *x, float *y, uint32_t rows, uint32_t nb, const float *bias,
                   const float *res, uint8_t *q8, void *stream) {
   NEED_OPEN();
@@ -1113,6 +1149,12 @@ static int gemv_x(int kind, const char *op, const void *w, const float *x, float
        14.1 / 16.3 / 22.9 against 16.6; 34816 x 5120 27.6 (8) against 21.9, 6144 x 5120 and the Q4_0
        shapes slower than their fused kernels, so only here. */
     rc = gemvk_launch(kind, w, x, 1, y, rows, nb, bias, res, q8, 8u, stream);
+    if (rc != -1) return rc;
+  }
+  /* not with y on x: there the workgroups would write what others still quantize */
+  if ((kind == AMDC_KIND_Q8_0 || kind == AMDC_KIND_Q6_K) && nb <= X8_FUSE_NB &&
+      ((uintptr_t)(y + rows) <= (uintptr_t)x || (uintptr_t)(x + 32u * (size_t)nb) <= (uintptr_t)y)) {
+    rc = gemvs8_launch(kind, w, x, 1, y, rows, nb, bias, res, q8, stream);
     if (rc != -1) return rc;
   }
   if (nb > x_fuse_nb || 320u * ng > GEMV_LDS_T1 || kind == AMDC_KIND_Q8_0 || kind == AMDC_KIND_Q6_K) {

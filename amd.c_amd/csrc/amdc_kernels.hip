@@ -502,6 +502,24 @@ __device__ __forceinline__ void load_item(Item &it, const uint8_t *wr, u32 ng, u
   for (u32 k = 0; k < 8u; k++) it.n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_nib_off(ng, g, k)));
 }
 
+template <int KIND>
+__device__ __forceinline__ void load_item(ItemQ8 &it, const uint8_t *wr, u32 ng, u32 g, bool ok) {
+  g = ok ? g : 0u;
+  it.h = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_header_off(g)));
+#pragma unroll
+  for (u32 k = 0; k < 16u; k++) it.n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_q8_off(ng, g, k)));
+}
+template <int KIND>
+__device__ __forceinline__ void load_item(ItemQ6 &it, const uint8_t *wr, u32 ng, u32 g, bool ok) {
+  g = ok ? g : 0u;
+  it.h = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_header_off(g)));
+  it.d = *(const unsigned short *)(wr + amdc_q6k_d_off(ng, g));
+#pragma unroll
+  for (u32 k = 0; k < 8u; k++) it.n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_q6k_nib_off(ng, g, k)));
+#pragma unroll
+  for (u32 k = 0; k < 4u; k++) it.x[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_q6k_hi_off(ng, g, k)));
+}
+
 // One super-group's contribution to a row: for each of its 8 blocks k (LDS
 // slot p = k GC + gl of the staged vector), the integer block dot and the
 // reference's per-block float step (src/cpu.c:81, 112, 142, 168).
@@ -558,7 +576,8 @@ __device__ __forceinline__ float item_dot(const typename ItemOf<KIND>::type &it,
 // unconditional (a block past nb reads the last block again and takes zeros),
 // so that no branch joins them. The max and the sum of a block's 8 lanes go
 // by DPP (xor 1, xor 2, then the half-row mirror).
-template <u32 NC, u32 NTH = NT> struct FusedQ8T {
+// HALF (Q6_K): instead of asum, 32 x the sum of each half of the block.
+template <u32 NC, u32 NTH = NT, bool HALF = false> struct FusedQ8T {
   static constexpr u32 BP = NTH / 8u; // blocks per pass
   u32 bp = BP;                         // ... at run time (a workgroup of blockDim.x < NTH threads: blockDim.x / 8)
   // a K range of the vector (the split-K kernels): super-groups sgb .. of the row go to LDS columns
@@ -592,11 +611,17 @@ template <u32 NC, u32 NTH = NT> struct FusedQ8T {
       u32 sum = (u32)qi[0] + (u32)qi[1] + (u32)qi[2] + (u32)qi[3];
       sum += (u32)__builtin_amdgcn_update_dpp(0, (int)sum, 0xB1, 0xF, 0xF, false);
       sum += (u32)__builtin_amdgcn_update_dpp(0, (int)sum, 0x4E, 0xF, 0xF, false);
+      const u32 half = sum;
       sum += (u32)__builtin_amdgcn_update_dpp(0, (int)sum, 0x141, 0xF, 0xF, false);
       if (b < nblk) {
         const u32 p = (b & 7u) * st + (b >> 3) - sgb;
         ((u32 *)(e < 4u ? &s_lo[p] : &s_hi[p]))[e & 3u] = word;
-        if (e == 0u) s_d[p] = d, s_as[p] = sum;
+        if (e == 0u) s_d[p] = d;
+        if constexpr (HALF) {
+          if ((e & 3u) == 0u) s_as[2u * p + (e >> 2)] = 32u * half;
+        } else {
+          if (e == 0u) s_as[p] = sum;
+        }
       }
       if (q8out && blockIdx.x == 0u && b < nb) { // the Q8 buffer, for other consumers
         ((u32 *)(q8out + 32u * b))[e] = word;
@@ -783,7 +808,7 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
   const u32 nth = QCN ? blockDim.x : NTH;
   const u32 ng = amdc_ngroups(nb), tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
   const u32 l = lane & (L - 1u), q = lane / L, rpw = 64u / L, rpg = (nth / 64u) * rpw;
-  const u64 RB = amdc_row_bytes(nb);
+  const u64 RB = amdc_row_bytes_k(KIND, nb);
   const u32 nblk = 8u * ng;
   u32x4 *s_lo = (u32x4 *)smem;
   u32x4 *s_hi = s_lo + nblk;
@@ -792,7 +817,8 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
   const u32 r = blockIdx.x * rpg + wv * rpw + q;
   const uint8_t *wr = W + (u64)(r < rows ? r : rows - 1u) * RB;
   constexpr u32 QC = QCN ? QCN : (QCH * NT) / NTH; // passes in flight: 128 blocks (QCN: QCN passes of nth / 8 blocks)
-  FusedQ8T<QC, NTH> fq;
+  constexpr bool H6 = KIND == AMDC_Q6_K; // the staged vector holds 32 x the sum of each half block
+  FusedQ8T<QC, NTH, H6> fq;
   fq.bp = nth / 8u;
   if (FQ) {
     fq.load(xf, nb, 0);
@@ -801,6 +827,10 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
   // the Q8 vector's first NSV chunks of the staging loop loaded ahead of the weights: loads complete in
   // issue order, so staged after them the vector waited for every weight load (MI355X: 5120 x 17408
   // Q4_K 19.7-20.1 -> 18.6-19.3 us; with 3 chunks, all of its 544 blocks, 14.8-15.2 -> 14.5 us)
+  auto put_as = [&](u32 p, const u32x4 &lo, const u32x4 &hi, u32 as, bool in) {
+    if constexpr (H6) ((u32x2 *)s_as)[p] = in ? (u32x2){32u * (u32)hsum16(lo), 32u * (u32)hsum16(hi)} : (u32x2)(0u);
+    else s_as[p] = in ? as : 0u;
+  };
   constexpr u32 NSV = NI >= 2u ? 3u : 2u;
   u32x4 vlo[NSV], vhi[NSV];
   float vd[NSV];
@@ -822,7 +852,7 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
   // loads issued first by all workgroups keep the memory busy meanwhile, and the items issued later
   // are not live during the quantization (the two-item Q4_0 kernel: 157 -> 126 VGPRs, 4 workgroups
   // per CU)
-  Item it[NI];
+  typename ItemOf<KIND>::type it[NI];
   constexpr u32 NI0 = FQ && NI >= 2u ? 1u : NI; // items issued before the quantization
   // Of the first item, only the header and PB nibble planes go out before the quantization (the rest
   // after it): the workgroup-per-CU kernels with one item per lane and the single-shot kernels with
@@ -862,7 +892,8 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
       if (j < nblk) {
         const u32 p = (j & 7u) * ng + (j >> 3);
         const bool in = j < nb;
-        s_lo[p] = in ? vlo[c] : (u32x4)(0u), s_hi[p] = in ? vhi[c] : (u32x4)(0u), s_d[p] = in ? vd[c] : 0.0f, s_as[p] = in ? vas[c] : 0u;
+        s_lo[p] = in ? vlo[c] : (u32x4)(0u), s_hi[p] = in ? vhi[c] : (u32x4)(0u), s_d[p] = in ? vd[c] : 0.0f;
+        put_as(p, vlo[c], vhi[c], vas[c], in);
       }
     }
     for (u32 j = tid + NSV * NTH; j < nblk; j += NTH) { // stage the rest of the Q8 vector (permuted)
@@ -876,7 +907,8 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
         d = ((const float *)(xq + 32u * nb))[j];
         as = ((const u32 *)(xq + 36u * nb))[j];
       }
-      s_lo[p] = lo, s_hi[p] = hi, s_d[p] = d, s_as[p] = as;
+      s_lo[p] = lo, s_hi[p] = hi, s_d[p] = d;
+      put_as(p, lo, hi, as, true);
     }
   }
   __syncthreads();
@@ -1232,6 +1264,16 @@ extern "C" __global__ __launch_bounds__(256) void amdc_gemv_q6_k_p2(const uint8_
                                                                    const float *bias, const float *res, u32 L) {
   gemv2_body<AMDC_Q6_K>(W, xq, y, rows, nb, bias, res, L);
 }
+// Q8_0 / Q6_K in the single-shot form (gemvs_body), on a Q8 and on an f32 vector: with a super-group's 17 or 14 loads
+// all out at once, 97 to 127 VGPRs hold 4 or 5 waves per SIMD where the form above holds two items and 2 waves.
+// Measured on MI355X (us, f32 vector: quantize launch and the form above / this): Q8_0 2048 x 2048 6.8 / 3.9, 11264 x
+// 2048 10.9 / 6.7, 32000 x 2048 16.5 / 12.7, 4096 x 4096 9.1 / 5.8; Q6_K 6144 x 2048 8.4 / 5.3, 1024 x 5120 6.9 / 5.6,
+// 4096 x 4096 8.8 / 5.9; with the quantize launch kept (long rows): Q8_0 4096 x 11008 14.8 / 13.4, 152064 x 5120 140 /
+// 127, Q6_K 4096 x 11008 14.5 / 12.1 (5120 x 17408 22.5 / 25.4, 152064 x 5120 110.7 / 117: not taken); on a Q8 vector
+// Q6_K 100000 x 2048 46.0 / 31.7, Q8_0 100000 x 2048 60.2 / 32.8, 36000 x 8192 51.6 / 45.7
+GEMVS_KERNELS(q8_0, AMDC_Q8_0, 1, s, 256)
+GEMVS_KERNELS(q6_k, AMDC_Q6_K, 1, s, 256)
+GEMVS_KERNELS(q8_0, AMDC_Q8_0, 2, s, 256)
 // the Q8_0 / Q6_K decode form with the fused RMSNorm tail (amdc_gemv_norm)
 #define GEMV2N_KERNEL(KN, KIND)                                                                                                      \
   extern "C" __global__ __launch_bounds__(256) void amdc_gemv_##KN##_pn(const uint8_t *W, const uint8_t *xq, float *y, u32 rows,    \

@@ -180,7 +180,8 @@ int amdc_gemv_q4_x(const void *w, const float *x, float *y, uint32_t rows, uint3
                    void *stream);
 int amdc_gemv_q4k_x(const void *w, const float *x, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res, uint8_t *q8,
                     void *stream);
-/* Q8_0 / Q6_K: always amdc_quant_q8 and the GEMV (two launches). */
+/* Q8_0 / Q6_K: one launch, every workgroup quantizing x, for nb <= 192 on
+ * matrices of up to some tens of thousand rows; else amdc_quant_q8 and the GEMV. */
 int amdc_gemv_q8_x(const void *w, const float *x, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res, uint8_t *q8,
                    void *stream);
 int amdc_gemv_q6k_x(const void *w, const float *x, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res, uint8_t *q8,
