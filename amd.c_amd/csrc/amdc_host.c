@@ -763,7 +763,7 @@ static int ws_take(size_t n, void **p);
 /* The verify GEMV on int8 MFMA (T <= 16): 64 rows per workgroup, K split
  * over aligned ranges of tiles (64 blocks each): for T <= 8 until the
  * workgroups fill the resident slots about once (Q4 kinds) or the CUs four
- * times (Q8_0, Q6_K), for T > 8 by an estimate of the time. A range holds S
+ * times (Q8_0), for T > 8 and Q6_K by an estimate of the time. A range holds S
  * tiles, S a power of two <= 4, so that its sum is a subtree of the
  * super-group tree (the kernels' order, equal to the decode GEMV's) and the
  * split sums' tree over the ranges (in the kernel for T <= 8, else
@@ -786,7 +786,7 @@ static int gemv8_launch(int kind, const void *w, const uint8_t *xq, float *y, ui
   if (want > 16u) want = 16u; /* amdc_gemm_reduce adds at most 16 ranges */
   u32 tps = 1;
   while (tps < 4u && tps * want < nt) tps <<= 1; /* the smallest S with ceil(nt / S) <= want (nt <= 32: S <= 2 for 16) */
-  if (T > 8u && t_ksplit <= 0 && wgs < 2u * cus) {
+  if (T > 8u && t_ksplit <= 0 && wgs < 2u * cus && kind != AMDC_KIND_Q6_K) {
     /* the 16-vector kernels hold one workgroup per CU: the range size S (1, 2, 4 tiles) with the fewest
        tile times, (rounds of workgroups) x S, plus one for the reduction launch of a split; ties to the
        larger S (grids of two workgroups per CU and more are not split). Measured on MI355X (T = 16, us): 11008 x 4096 Q4_0 16.7 unsplit against 20.8 in 2 splits,
@@ -807,6 +807,21 @@ static int gemv8_launch(int kind, const void *w, const uint8_t *xq, float *y, ui
   /* T <= 8, 2 tiles of K and at least half a workgroup per CU: unsplit (MI355X, T = 8, us: 11008 x
      4096 Q8_0 14.3 against 15.2-15.4 in 2 splits, Q4_0 12.2 against 12.3) */
   if (T <= 8u && nt == 2u && t_ksplit <= 0 && 2u * wgs >= cus) tps = 2u;
+  if (kind == AMDC_KIND_Q6_K && t_ksplit <= 0) {
+    /* Q6_K, any T: two workgroups per CU; the range size S with the fewest tile times, rounds (at least one, else
+       as many as the workgroups are of the resident ones) x S, plus one for a split's sums; ties to the smaller S.
+       Measured on MI355X (us, S = 1, 2, 4, T = 16): 5120 x 17408 35.7 / 36.7 / 50.9, 17408 x 5120 37.4 / 37.7 / 46.6,
+       20480 x 8192 52 / 57 / 62, 32000 x 4096 42 / 34 unsplit, 11008 x 4096 22 / 26.7 unsplit; T = 8 alike */
+    const double slots = 2.0 * cus;
+    double best = 1e30;
+    tps = 4u;
+    for (u32 S = 4u; S >= 1u && wgs < 2u * cus; S >>= 1) {
+      const u32 n = (nt + S - 1u) / S;
+      if (n > 16u) break;
+      const double r = (double)wgs * n / slots, est = (r > 1.0 ? r : 1.0) * (S < nt ? S : nt) + (n > 1u ? 1.0 : 0.0);
+      if (est <= best) best = est, tps = S;
+    }
+  }
   const u32 ks = (nt + tps - 1u) / tps;
   float *part = NULL;
   if (ks > 1u) {
@@ -968,12 +983,14 @@ static int gemv_launch(int kind, const void *w, const uint8_t *xq, float *y, uin
       while (L < 64u && L < ng) L <<= 1;
       const u32 ni = (ng + L - 1u) / L, rpg = 4u * (64u / L), nrg = (rows + rpg - 1u) / rpg;
       const u64 rb = amdc_row_bytes_k(kind, nb);
-      /* measured on MI355X (us, this kernel / the MFMA verify kernel): Q6_K 1024 x 5120 T = 2, 4, 8 5.2 /
-         14.3, 6.9 / 14.4, 10.3 / 17.8; 4096 x 4096 6.6 / 15.4, 8.2 / 15.4, 11.5 / 18.6; 6144 x 5120 T = 4
-         15.7 / 17.2. Q8_0 4096 x 4096 6.4 / 9.5, 7.8 / 9.6, 10.6 / 10.1; 11008 x 4096 T = 2, 4 12.3 /
+      /* measured on MI355X (us, this kernel / the MFMA verify kernel): Q6_K 1024 x 5120 T = 2, 4, 8 5.5 /
+         10.9, 7.1 / 10.8, 10.5 / 11.3; 4096 x 4096 6.8 / 12.1, 8.5 / 12.2, 11.7 / 12.7; 6144 x 5120 T = 4, 6
+         15.5 / 15.8, 18.7 / 16.2; 11008 x 4096 T = 4 16.8 / 17.1; 4096 x 11008 (43 of 64 lanes) T = 4 21.0 /
+         17.6; 17408 x 5120 T = 2 25.1 / 28.7: Q6_K past T = 2 counts its idle lanes too. Q8_0 4096 x 4096 6.4 / 9.5, 7.8 / 9.6, 10.6 / 10.1; 11008 x 4096 T = 2, 4 12.3 /
          15.2, 15.4 / 14.9; 1024 x 2048 T = 8 7.6 / 6.5: Q8_0 only up to T = 4 and half the size */
       const u64 lim = kind == AMDC_KIND_Q6_K ? M8_MAX : T <= 4u ? M8_MAX * 2u / 3u : 0u;
-      if (ni == 1u && lds <= 64u * 1024u && (u64)T * rows * ng <= lim && (u64)rows * rb + rb < (1ull << 32)) {
+      const u32 gl = kind == AMDC_KIND_Q6_K && T > 2u ? L : ng;
+      if (ni == 1u && lds <= 64u * 1024u && (u64)T * rows * gl <= lim && (u64)rows * rb + rb < (1ull << 32)) {
         void *a[] = {&w, &xq, &y, &rows, &nb, &bias, &res, (void *)&L, &T, &xs, &ys, &rs};
         return launch(K_GEMVM8 + (kind == AMDC_KIND_Q6_K ? 1 : 0), nrg, 1, lds, stream, a);
       }

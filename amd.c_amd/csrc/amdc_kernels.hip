@@ -3836,51 +3836,46 @@ extern "C" __global__ __launch_bounds__(256) void amdc_gemv_q8_0_v16(const uint8
   gemv8_body<AMDC_Q8_0, 1, 2, 1>(W, xq, y, rows, nb, bias, res, T, xs, ys, rs, part, tps, cnt);
 }
 
-// The verify GEMV for Q6_K (T <= 8). A Q6_K weight's scale changes every 16
-// weights, so each K quarter of v_mfma_i32_16x16x64_i8 is one half sub-block
-// and each of the 16 columns one (quarter, token) pair:
-//   A (16 rows x 64): lane (row i, h) = q - 32 of the 16 weights of half h & 1
-//     of sub-block (g + h / 2, k) (a pair of super-groups, one plane, as the Q4
-//     pair kernel): its 16 nibble bytes and its half's high-bit word, then
-//     ((v | 0x80) - 0x20) ^ 0x80 per byte
-//   B (64 x 16 columns n = 4 q + t): the 16 activations of quarter q for token
-//     t (4 tokens per MFMA, two MFMAs for 8), zeros in the other quarters (LDS
-//     holds only the nonzero quarter of each column; the other lanes use 0)
-// so that C[r][4 q + t] is the exact half dot sum (q - 32) a of ie_q6k_dots for
-// quarter q. The float steps are the decode GEMV's, in its order (bit-equal to
-// it): the lanes of quarter 0 (2) take quarter 1's (3's) dot from the lane 4
-// columns up and apply leaf = fma(fma(s1, d1, s0 d0), d_a, leaf) per block
-// (src/cpu.c:142, s = d sc), a leaf per super-group; the tile's 8 leaves join
-// as ((g0 + g1) + (g2 + g3)) + ... (row_ror:8 for the pairs), and the tiles of
-// a range and the ranges as gemv8_body's (the super-group tree).
-// Tiles of 8 super-groups as gemv8_body: activations and d_a staged in LDS in
-// B form. The weights go into LDS as in gemv8_body, in whole 128-byte lines: a
-// ring step is the nibble planes 2m, 2m + 1 and high-bit plane m of the wave's
-// 16 rows (6 KB), 2 steps per wave. The scales: each wave's table of the int8
-// sc per (sub-block, half, row) and d per (super-group, row); s = d sc (exact).
-// Split K over gridDim.y.
-template <int NQ, int NS>
+// The verify GEMV for Q6_K (T <= 16), in the manner of gemv8_body with one wave per 16 rows. A Q6_K weight's
+// scale changes every 16 weights, so a block has two dots, and each K quarter of v_mfma_i32_16x16x64_i8 is one
+// half sub-block:
+//   A (16 rows x 64): lane (row i, h) = 4 (q - 32) of the 16 weights of half h & 1 of sub-block (g + h / 2, k), as
+//     int8: the 4 low bits of a weight at bits 2 .. 5 of its byte (a rotation of the nibble dword), the high two at
+//     6 and 7, the top one inverted
+//   B (64 x 16 columns n = t + 8 pp): token t's 16 activations of quarter 2 pp + e, zeros in the other quarters,
+//     once for each half e (the LDS holds the halves; the lanes of other quarters take zeros by a mask)
+// so that the two products' C[r][t + 8 pp] are 4 times the exact half dots of ie_q6k_dots of block (g + pp, k), in
+// one lane, for 8 tokens. The float steps are the decode GEMV's, in its order (bit-equal to it): leaf = fma(fma(s1, d1,
+// s0 d0), d_a, leaf) per block (src/cpu.c:142, s = d sc; here s / 4, exact, and 4 d), a leaf per super-group; the
+// leaves of a tile, the tiles of a range and the ranges as gemv8_body's (the super-group tree).
+// A ring step is the nibble planes 2m, 2m + 1 and high-bit plane m of the wave's 16 rows (6 KB). Each
+// wave builds the scales s / 4 of its rows plane by plane, as gemv8_body. Split K over gridDim.y.
+// What bounds it is the issue of vector instructions, 1681 per wave and tile at T <= 8 where one product with columns
+// (quarter, token) for 4 tokens, whose halves met by DPP in half the lanes, took 3428; then a tile's chain of loads, two
+// waves per SIMD. Measured on MI355X (us, that form / this): T = 8 5120 x 17408 37.6 / 27.3, 17408 x 5120 38.0 / 29.9,
+// 4096 x 11008 24.8 / 17.9, 32000 x 4096 39.0 / 28.1, 152064 x 5120 221 / 164 (T = 2 182 / 157); T = 16 (one workgroup per
+// CU / two) 81 / 35, 87 / 37, 51 / 22, 97 / 35, 591 / 218.
+template <int NH, int NS>
 __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, const uint8_t *__restrict__ xq, float *__restrict__ y,
                                                u32 rows, u32 nb, const float *__restrict__ bias, const float *__restrict__ res, u32 T,
                                                u32 xs, u32 ys, u32 rs, float *__restrict__ part, u32 tps, u32 *__restrict__ arrive) {
-  constexpr u32 NTK = 4u * NQ; // tokens per launch: NQ groups of 4
+  constexpr u32 NTK = 8u * NH; // tokens per launch: NH halves of 8
+  constexpr u32 CH = 128u;     // u32x4 per 2 KB chunk (16 rows x 128 bytes)
   typedef __attribute__((address_space(3))) void lds_t;
-  constexpr u32 CH = 128u; // u32x4 per 2 KB chunk (16 rows x 128 bytes)
   __shared__ __attribute__((aligned(16))) u32x4 sw0[4][3u * CH]; // per wave: nibble planes 2m, 2m + 1, high plane m
   __shared__ __attribute__((aligned(16))) u32x4 sw1[NS > 1 ? 4 : 1][NS > 1 ? 3u * CH : 1u];
-  __shared__ __attribute__((aligned(16))) u32x4 sB[NQ][32][16]; // [token group][pair p + 4 k][column]: the column's nonzero quarter
+  __shared__ __attribute__((aligned(16))) u32x4 sB[NH][32][2][16]; // [token half][pair p + 4 k][half e][column, swizzled]
   __shared__ __attribute__((aligned(16))) float sda[64][NTK];      // d_a [sub-block][token]
-  __shared__ __attribute__((aligned(16))) uint8_t ssc[4][64][2][16]; // per wave: the int8 sc [sub-block][half][row]
-  __shared__ __attribute__((aligned(16))) float sd[4][8][16];        // per wave: d [super-group][row]
-  const u32 ng = nb >> 3, nt = (ng + 7u) >> 3, tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-  const u32 i16 = lane & 15u, h = lane >> 4, n = i16, qn = n >> 2, tq = n & 3u;
+  __shared__ __attribute__((aligned(16))) float ssc[4][2][2][8][16]; // per wave and plane (double-buffered): s / 4 [half][super-group][row]
+  const u32 ng = nb >> 3, nt = (ng + 7u) >> 3, tid = threadIdx.x, lane = tid & 63u, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const u32 i16 = lane & 15u, h = lane >> 4, n = i16, tk = n & 7u, pp = n >> 3;
   const u32 RB = (u32)amdc_q6k_row_bytes(nb), D = amdc_q6k_dpad(ng);
   const u32 rt0 = blockIdx.x * 64u, r0 = rt0 + 16u * w;
   auto clamp_row = [&](u32 r) { return (r < rows ? r : rows - 1u) - rt0; };
   const __amdgpu_buffer_rsrc_t rw = rsrc(W + (u64)rt0 * RB, (u32)min((u64)(rows - rt0) * RB, (u64)0xFFFFFFF0u));
   const u32 wo = clamp_row(r0 + i16) * RB;
   const u32 wl0 = clamp_row(r0 + (lane >> 3)) * RB, wl1 = clamp_row(r0 + 8u + (lane >> 3)) * RB; // the plane loads' rows
-  const u32 lcol = lane & 7u, g0 = lcol ^ v8_swz(lane >> 3), g1 = lcol ^ v8_swz(8u + (lane >> 3));
+  const u32 g0 = (lane & 7u) ^ v8_swz(lane >> 3), g1 = (lane & 7u) ^ v8_swz(8u + (lane >> 3));    // and super-groups
   const __amdgpu_buffer_rsrc_t rxq = rsrc(xq, (u32)min((u64)T * xs, (u64)0xFFFFFFF0u));
   constexpr u32 OOB = 0xFFFFFFF0u;
   const u32 ks = blockIdx.y, t0 = ks * tps, t1 = t0 + tps < nt ? t0 + tps : nt;
@@ -3889,10 +3884,8 @@ __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, co
     if (s == 0u || NS == 1) return sw0[w];
     return sw1[NS > 1 ? w : 0u];
   };
-  // step m of tile t into slot s (off: every load out of range). The slot was read by the planes just
-  // before: the wave's LDS reads are complete (lgkmcnt 0) and ordered before the refill (the compiler
-  // does not order LDS reads against these loads into the LDS; with a ring of one step the last reads
-  // sit right before the refill)
+  // step m of tile t into slot s (off: every load out of range, zeros). The wave's reads of the slot's step before
+  // are complete (lgkmcnt 0) and ordered before the refill (the fences)
   auto issue = [&](u32 t, u32 m, u32 s, bool on) {
     const u32 gt = on ? gtile(t) : 0u;
     __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
@@ -3900,31 +3893,28 @@ __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, co
 #pragma unroll
     for (u32 c = 0; c < 3u; c++) {
       const u32 base = c < 2u ? 16u * ng + D + 1024u * t + 16u * (2u * m + c) * gt : 144u * ng + D + 512u * t + 16u * m * gt;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_t *)(slot(s) + CH * c), 16, g0 < gt ? wl0 + base + 16u * g0 : OOB, 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_t *)(slot(s) + CH * c + 64u), 16, g1 < gt ? wl1 + base + 16u * g1 : OOB, 0, 0, 0);
+      lds_load16(rw, (lds_t *)(slot(s) + CH * c), g0 < gt ? wl0 + base + 16u * g0 : OOB);
+      lds_load16(rw, (lds_t *)(slot(s) + CH * c + 64u), g1 < gt ? wl1 + base + 16u * g1 : OOB);
     }
     __asm__ volatile("" ::: "memory");
   };
-  u32x4 ra4[2 * NQ];
-  float rd[NQ];
-  u32x4 rh[2];
-  u32 rdd[2];
-  // the tile's activations, d_a and headers into registers (on false: every load past the resource,
-  // zeros, so that the loads in flight count statically)
-  constexpr u32 NFT = 3u * NQ + 4u; // its loads
+  constexpr u32 NC4 = 4u * NH, NCS = 2u * NH, NFT = NC4 + NCS + 4u; // halves and d_a per thread; loads of fetch_tile
+  u32x4 ra4[NC4], rh[2];
+  float rd[NCS];
+  u32 rdd[2]; // the headers and d of row i16, super-groups h and h + 4 of the tile
+  // the tile's activations, d_a and headers into registers (off: every load past the resource, zeros, so that the
+  // loads in flight count statically)
   auto fetch_tile = [&](u32 t, bool on) {
     const u32 gt = on ? gtile(t) : 0u;
 #pragma unroll
-    for (u32 c = 0; c < 2u * NQ; c++) {
+    for (u32 c = 0; c < NC4; c++) {
       const u32 i = tid + c * NT, half = i & 1u, bl = (i >> 1) & 63u, tok = i >> 7, b = 64u * t + bl;
-      const bool ok = tok < T && (bl >> 3) < gt;
-      ra4[c] = __builtin_amdgcn_raw_buffer_load_b128(rxq, ok ? tok * xs + 32u * b + 16u * half : OOB, 0, 0);
+      ra4[c] = __builtin_amdgcn_raw_buffer_load_b128(rxq, tok < T && (bl >> 3) < gt ? tok * xs + 32u * b + 16u * half : OOB, 0, 0);
     }
 #pragma unroll
-    for (u32 c = 0; c < (u32)NQ; c++) {
+    for (u32 c = 0; c < NCS; c++) {
       const u32 i = tid + c * NT, tok = i & (NTK - 1u), bl = i / NTK, b = 64u * t + bl;
-      const bool ok = tok < T && (bl >> 3) < gt;
-      rd[c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rxq, ok ? tok * xs + 32u * nb + 4u * b : OOB, 0, 0));
+      rd[c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rxq, tok < T && (bl >> 3) < gt ? tok * xs + 32u * nb + 4u * b : OOB, 0, 0));
     }
 #pragma unroll
     for (u32 q = 0; q < 2u; q++) {
@@ -3933,90 +3923,81 @@ __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, co
       rdd[q] = __builtin_amdgcn_raw_buffer_load_b16(rw, gl < gt ? wo + (u32)amdc_q6k_d_off(ng, g) : OOB, 0, 0);
     }
   };
+  u32x4 hc[2]; // the current tile's headers and d / 4
+  float dq[2] = {};
+  auto scales = [&](u32 k) { // plane k's table, this lane's entries: d sc / 4, exact (an f16 times an int8)
+#pragma unroll
+    for (u32 q = 0; q < 2u; q++) {
+      const u32 sc = hword(hc[q], k >> 1) >> (16u * (k & 1u));
+#pragma unroll
+      for (u32 e = 0; e < 2u; e++) ssc[w][k & 1u][e][h + 4u * q][i16] = dq[q] * (float)(int)(int8_t)(sc >> (8u * e));
+    }
+  };
   auto stage_tile = [&]() {
 #pragma unroll
-    for (u32 c = 0; c < 2u * NQ; c++) { // (half, sub-block (gl, k), token) -> quarter 2 (gl & 1) + half of pair gl / 2
+    for (u32 c = 0; c < NC4; c++) { // (half, sub-block (gl, k), token): column token % 8 + 8 (gl & 1)
       const u32 i = tid + c * NT, half = i & 1u, bl = (i >> 1) & 63u, tok = i >> 7, gl = bl >> 3, k = bl & 7u;
-      const u32 q = 2u * (gl & 1u) + half;
-      sB[tok >> 2][(gl >> 1) + 4u * k][4u * q + (tok & 3u)] = ra4[c];
+      sB[tok >> 3][(gl >> 1) + 4u * k][half][((tok & 7u) + 8u * (gl & 1u)) ^ v8_bswz(k, half)] = ra4[c];
     }
 #pragma unroll
-    for (u32 c = 0; c < (u32)NQ; c++) {
+    for (u32 c = 0; c < NCS; c++) {
       const u32 i = tid + c * NT;
       sda[i / NTK][i % NTK] = rd[c];
     }
 #pragma unroll
-    for (u32 q = 0; q < 2u; q++) { // this wave's tables: row i16, super-groups h, h + 4
-      const u32 gl = h + 4u * q;
-      sd[w][gl][i16] = h2f(rdd[q]);
-#pragma unroll
-      for (u32 k = 0; k < 8u; k++)
-#pragma unroll
-        for (u32 e = 0; e < 2u; e++)
-          ssc[w][8u * gl + k][e][i16] = (uint8_t)(hword(rh[q], k >> 1) >> (16u * (k & 1u) + 8u * e));
-    }
+    for (u32 q = 0; q < 2u; q++) hc[q] = rh[q], dq[q] = 0.25f * h2f(rdd[q]);
+    scales(0u);
   };
-  float lf[NQ][4][4]; // the leaves: [token group][pair p: super-group 2 p + qn / 2 (lanes of an even quarter qn)][row 4 h + v]
-  const u32 nth = (T + 3u) >> 2; // token groups with tokens (group 0 always: T >= 1)
-  // the MFMAs of plane k = 2 m + e from slot s
-  auto plane = [&](u32 m, u32 e, u32 npair, u32 s) {
+  float lf[NH][4][4]; // the leaves: [token half][pair p: super-group 2 p + pp][row 4 h + v]
+  const u32 rot = (h & 1u) ? 2u : 30u;                                       // a nibble to bits 2 .. 5 of its byte
+  const u32 m0 = h == 2u * pp ? ~0u : 0u, m1 = h == 2u * pp + 1u ? ~0u : 0u; // this lane's B operand of half 0, of half 1
+  // lane offsets, opaque, so that the planes' and pairs' constants go into the reads' offset fields
+  u32 oda = 4u * (8u * pp * NTK + tk), osc = 4u * (16u * pp + 4u * h), ohi = 4u * (h & 1u);
+  __asm__("" : "+v"(oda), "+v"(osc), "+v"(ohi));
+  auto at = [](const void *p, u32 o) { return (const uint8_t *)p + o; };
+  // plane k = 2 m + e from slot s: the next pair's (NH = 2: token half's) MFMAs go out before a pair's results are
+  // used. A partial tile's missing super-groups are zeros, as in gemv8_body
+  auto plane = [&](u32 m, u32 e, u32 s) {
     const u32 k = 2u * m + e;
     const u32x4 *sl = slot(s);
-    v4i c[NQ][2];
-    const u32 sft = 4u * (h & 1u);
-    auto mfma = [&](u32 p) {
-      const u32 col = (2u * p + (h >> 1)) ^ v8_swz(i16);
-      const u32x4 wq = sl[CH * e + 8u * i16 + col];
-      const u32 hq = ((const u32 *)(sl + 2u * CH + 8u * i16 + col))[2u * e + (h & 1u)];
-      u32 a[4];
+    v4i c[2][2], av;
+    auto mfma = [&](u32 u) {
+      const u32 p = u / NH, th = u % NH;
+      if (th == 0u) {
+        const u32 col = 8u * i16 + ((2u * p + (h >> 1)) ^ v8_swz(i16));
+        const u32x4 wq = sl[CH * e + col];
+        const u32 hq = *(const u32 *)at(&sl[2u * CH], 16u * col + ohi + 8u * e) ^ 0xAAAAAAAAu;
 #pragma unroll
-      for (u32 i = 0; i < 4u; i++) {
-        const u32 v = ((wq[i] >> sft) & 0x0F0F0F0Fu) | (((hq >> (2u * i)) & 0x03030303u) << 4);
-        a[i] = ((v | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
-      }
-      const v4i av = {(int)a[0], (int)a[1], (int)a[2], (int)a[3]};
-#pragma unroll
-      for (u32 th = 0; th < (u32)NQ; th++)
-        if (th == 0u || th < nth)
-          c[th][p & 1u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, h == qn ? __builtin_bit_cast(v4i, sB[th][p + 4u * k][n]) : (v4i){0, 0, 0, 0},
-                                                                 (v4i){0, 0, 0, 0}, 0, 0, 0);
-    };
-    // pair p + 1's MFMAs go out before pair p's results are used (two result sets live)
-    mfma(0u);
-#pragma unroll
-    for (u32 p = 0; p < 4u; p++) {
-      if (p >= npair) break;
-      if (p + 1u < npair) mfma(p + 1u);
-      // the lanes of an even quarter qn (half 0 of super-group 2 p + qn / 2) take half 1's dot from the
-      // lane 4 columns up (row_ror:12) and apply the decode GEMV's block step, src/cpu.c:142:
-      // leaf = fma(fma(s1, d1, s0 d0), d_a, leaf), s = d sc (the lanes of odd quarters compute unused values)
-      const u32 bl = 8u * (2u * p + (qn >> 1)) + k; // this lane's sub-block
-      // d of this lane's 4 rows, read per pair (kept in registers for the 4 pairs it costs the kernel the
-      // 256-VGPR limit of two waves per SIMD: 264 VGPRs)
-      const v4f dp = *(const v4f *)&sd[w][2u * p + (qn >> 1)][4u * h];
-      const u32 sc0 = *(const u32 *)&ssc[w][bl][0][4u * h], sc1 = *(const u32 *)&ssc[w][bl][1][4u * h];
-      v4f s0, s1;
-#pragma unroll
-      for (u32 v = 0; v < 4u; v++) {
-        s0[v] = dp[v] * (float)(int)(int8_t)(sc0 >> (8u * v)); // d sc, exact (as the decode GEMV's dsc * sc)
-        s1[v] = dp[v] * (float)(int)(int8_t)(sc1 >> (8u * v));
-      }
-#pragma unroll
-      for (u32 th = 0; th < (u32)NQ; th++) {
-        if (th > 0u && th >= nth) break;
-        const float da = sda[bl][tq + 4u * th];
-#pragma unroll
-        for (u32 v = 0; v < 4u; v++) {
-          const int d0 = c[th][p & 1u][v], d1 = __builtin_amdgcn_update_dpp(0, d0, 0x12C, 0xF, 0xF, false); // row_ror:12: column n + 4
-          lf[th][p][v] = __builtin_fmaf(__builtin_fmaf(s1[v], (float)d1, s0[v] * (float)d0), da, lf[th][p][v]);
+        for (u32 i = 0; i < 4u; i++) {
+          const u32 lo = __builtin_amdgcn_alignbit(wq[i], wq[i], rot), hi = hq << (6u - 2u * i);
+          av[i] = (int)((lo & 0x3C3C3C3Cu) | (hi & 0xC0C0C0C0u));
         }
       }
+      const u32x4 b = sB[th][p + 4u * k][h & 1u][n ^ v8_bswz(k, h)];
+      c[u & 1u][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, __builtin_bit_cast(v4i, b & m0), (v4i){0, 0, 0, 0}, 0, 0, 0);
+      c[u & 1u][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, __builtin_bit_cast(v4i, b & m1), (v4i){0, 0, 0, 0}, 0, 0, 0);
+    };
+    mfma(0u);
+#pragma unroll
+    for (u32 u = 0; u < 4u * NH; u++) {
+      if (u + 1u < 4u * NH) mfma(u + 1u);
+      if (u == 0u && k + 1u < 8u) scales(k + 1u); // the next plane's table, while the MFMAs run
+      const u32 p = u / NH, th = u % NH; // this lane's super-group is 2 p + pp
+      const v4f s0 = *(const v4f *)at(&ssc[w][k & 1u][0][2u * p], osc), s1 = *(const v4f *)at(&ssc[w][k & 1u][1][2u * p], osc);
+      const float da = *(const float *)at(&sda[16u * p + k][8u * th], oda);
+#pragma unroll
+      for (u32 v = 0; v < 4u; v++)
+        lf[th][p][v] = __builtin_fmaf(__builtin_fmaf(s1[v], (float)c[u & 1u][1][v], s0[v] * (float)c[u & 1u][0][v]), da, lf[th][p][v]);
+      if (NH > 1) __builtin_amdgcn_sched_barrier(0); // (registers)
     }
   };
+  // t1 again, out of the compiler's sight: each plane a block of its own, or the results of many wait in registers
+  u32 tx = t1;
+  __asm__("" : "+s"(tx));
   // the tree over the range's tiles, as gemv8_body: st[j] a pending subtree of 2^j tiles, out the range's sum
-  float st[2][NQ][4], out[NQ][4];
+  float st[2][NH][4], out[NH][4];
 #pragma unroll
-  for (u32 th = 0; th < (u32)NQ; th++)
+  for (u32 th = 0; th < (u32)NH; th++)
 #pragma unroll
     for (u32 v = 0; v < 4u; v++) out[th][v] = 0.0f, st[0][th][v] = st[1][th][v] = 0.0f;
   if (t0 < t1) {
@@ -4026,41 +4007,37 @@ __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, co
   }
   for (u32 t = t0; t < t1; t++) {
     const bool more = t + 1u < t1;
-    const u32 npair = (gtile(t) + 1u) >> 1;
     v8_barrier(); // the previous tile's readers are done
     stage_tile();
     v8_barrier();
 #pragma unroll
-    for (u32 th = 0; th < (u32)NQ; th++)
+    for (u32 th = 0; th < (u32)NH; th++)
 #pragma unroll
       for (u32 p = 0; p < 4u; p++)
 #pragma unroll
         for (u32 v = 0; v < 4u; v++) lf[th][p][v] = 0.0f;
 #pragma unroll
     for (u32 m = 0; m < 4u; m++) {
-      // step m's loads into its slot have landed: issued after them, in this fixed order, are the next
-      // step's 6 (NS = 2) and, for steps 1 and 2 (NS = 2) or 1 (NS = 1), the next tile's activation loads
-      // (issued after step 0). The compiler's own waits are not relied on: it takes a 1 KB load into the
-      // LDS for a 16-byte store and moved the high-bit word read of a freshly refilled slot above its
-      // wait (with a one-step ring that read the previous step's bits)
-      vm_wait(NS == 2 ? 6u + (m == 1u || m == 2u ? NFT : 0u) : (m == 1u ? NFT : 0u));
-      plane(m, 0u, npair, m % (u32)NS);
-      plane(m, 1u, npair, m % (u32)NS);
+      // step m's loads into its slot have landed: issued after them are the NS - 1 later steps' and, for steps 1 ..
+      // NS, the next tile's activation loads (issued after step 0)
+      vm_wait((NS - 1u) * 6u + (m > 0u && m <= (u32)NS ? NFT : 0u));
+      if (t < tx) plane(m, 0u, m % (u32)NS);
+      if (t < tx) plane(m, 1u, m % (u32)NS);
       // issued also after the range's last tile (as zeros), so that the waits count statically
       if (m + (u32)NS < 4u) issue(t, m + (u32)NS, m % (u32)NS, true);
       else issue(t + 1u, m + (u32)NS - 4u, m % (u32)NS, more);
       if (m == 0u) fetch_tile(t + 1u, more); // in flight during this tile (issued also past the range)
     }
-    // the tile's subtree: super-groups (2 p, 2 p + 1) from quarters 0 and 2 (row_ror:8), then ((0 + 1) + (2 + 3)),
+    // the tile's subtree: super-groups (2 p, 2 p + 1) across the two columns (row_ror:8), then ((0 + 1) + (2 + 3)),
     // then into the tree over tiles (c: the tiles before this one in the range)
     const u32 c = t - t0;
 #pragma unroll
-    for (u32 th = 0; th < (u32)NQ; th++)
+    for (u32 th = 0; th < (u32)NH; th++)
 #pragma unroll
       for (u32 v = 0; v < 4u; v++) {
         float pr[4];
 #pragma unroll
-        for (u32 p = 0; p < 4u; p++) pr[p] = lf[th][p][v] + dpp<0x128>(lf[th][p][v]); // row_ror:8
+        for (u32 p = 0; p < 4u; p++) pr[p] = lf[th][p][v] + dpp<0x128>(lf[th][p][v]);
         float xv = (pr[0] + pr[1]) + (pr[2] + pr[3]);
         if (c & 1u) {
           xv = st[0][th][v] + xv;
@@ -4075,31 +4052,25 @@ __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, co
   const u32 cnt = t1 > t0 ? t1 - t0 : 0u;
   if (cnt < 4u) {
 #pragma unroll
-    for (u32 th = 0; th < (u32)NQ; th++)
+    for (u32 th = 0; th < (u32)NH; th++)
 #pragma unroll
       for (u32 v = 0; v < 4u; v++) out[th][v] = cnt == 3u ? st[1][th][v] + st[0][th][v] : cnt == 2u ? st[1][th][v] : st[0][th][v];
   }
-  float acc[NQ][4];
 #pragma unroll
-  for (u32 th = 0; th < (u32)NQ; th++)
-#pragma unroll
-    for (u32 v = 0; v < 4u; v++) acc[th][v] = out[th][v];
-  if (qn == 0u) {
-#pragma unroll
-    for (u32 th = 0; th < (u32)NQ; th++) {
-      const u32 tk = tq + 4u * th;
-      if (tk >= T) continue;
+  for (u32 th = 0; th < (u32)NH; th++) {
+    const u32 tt = tk + 8u * th;
+    if (pp == 0u && tt < T) {
 #pragma unroll
       for (u32 v = 0; v < 4u; v++) {
         const u32 r = r0 + 4u * h + v;
         if (r >= rows) continue;
         if (part) {
-          split_put(&part[((u64)ks * T + tk) * rows + r], acc[th][v]);
+          split_put(&part[((u64)ks * T + tt) * rows + r], out[th][v]);
         } else {
-          float o = acc[th][v];
+          float o = out[th][v];
           if (bias) o = o + bias[r];
-          if (res) o = res[(u64)tk * rs + r] + o;
-          y[(u64)tk * ys + r] = o;
+          if (res) o = res[(u64)tt * rs + r] + o;
+          y[(u64)tt * ys + r] = o;
         }
       }
     }
@@ -4111,11 +4082,11 @@ __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, co
 extern "C" __global__ __launch_bounds__(256) void amdc_gemv_q6_k_v8(const uint8_t *W, const uint8_t *xq, float *y, u32 rows, u32 nb,
                                                                    const float *bias, const float *res, u32 T, u32 xs, u32 ys, u32 rs,
                                                                    float *part, u32 tps, u32 *cnt) {
-  gemv8_q6k_body<2, 2>(W, xq, y, rows, nb, bias, res, T, xs, ys, rs, part, tps, cnt);
+  gemv8_q6k_body<1, 2>(W, xq, y, rows, nb, bias, res, T, xs, ys, rs, part, tps, cnt);
 }
-// up to 16 vectors: four token groups per A operand, a ring of one step (72 KB of LDS, 2 workgroups per CU)
-extern "C" __global__ __launch_bounds__(256) void amdc_gemv_q6_k_v16(const uint8_t *W, const uint8_t *xq, float *y, u32 rows, u32 nb,
+// up to 16 vectors: two token halves per A operand, a ring of one step (2 workgroups per CU)
+extern "C" __global__ __launch_bounds__(256, 2) void amdc_gemv_q6_k_v16(const uint8_t *W, const uint8_t *xq, float *y, u32 rows, u32 nb,
                                                                     const float *bias, const float *res, u32 T, u32 xs, u32 ys, u32 rs,
                                                                     float *part, u32 tps, u32 *cnt) {
-  gemv8_q6k_body<4, 1>(W, xq, y, rows, nb, bias, res, T, xs, ys, rs, part, tps, cnt);
+  gemv8_q6k_body<2, 1>(W, xq, y, rows, nb, bias, res, T, xs, ys, rs, part, tps, cnt);
 }
