@@ -3154,8 +3154,10 @@ __device__ __forceinline__ void a_frag_w6(u32 q0, u32 q1, h2 s, h8 &hi, h8 &lo) 
 //   Q4_0, Q8_0: acc_rt += (d_rb da_tb) X_rtb
 // What bounds it is the issue of vector instructions (4 cycles each, an MFMA 8; measured): one fma per element and
 // block, the A operands, and waits. So:
-// - a wave takes 64 rows x 32 NJ tokens in 32 x 32 tiles: an A operand (9 instructions per 8 weights) serves 64
-//   tokens where gemmh's serves 32, and half as many MFMAs are issued as in 16 x 16 tiles;
+// - a wave takes 64 rows x 64 tokens in 32 x 32 tiles, or 32 x 64 where the tile has 64 tokens: an A operand (9
+//   instructions per 8 weights) serves 64 tokens where gemmh's serves 32, and half as many MFMAs are issued as in 16 x 16
+//   tiles (64-token tiles as 64 rows x 32 tokens per wave, us, that / this: 17408 x 5120 Q4_K T = 64 56.5 / 51.5, 11008 x
+//   4096 Q4_0 T = 77 44.6 / 42.7, 11008 x 4096 Q6_K T = 64 40.8 / 38.4);
 // - everything comes into the LDS by loads that touch no register, a stage of two blocks at a time, a stage or two
 //   ahead, one barrier per stage; the activations as prepared images of it, so that every read of it is 16
 //   consecutive bytes per lane;
@@ -3182,6 +3184,8 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
   constexpr u32 TW = 64u * NJ, SB = gw_stage(Q4K, TW), NB = SB / 1024u; // a stage's image, in 1 KB loads
   constexpr u32 NF = NB / 4u, NR = NB % 4u;                            // whole rounds of the group's 4 waves, and the rest
   constexpr u32 NA = Q8 ? 8u : 4u, NX = Q6 ? 2u : 0u, OA = NB * 1024u, OX = OA + NA * 1024u, STAGE = OX + NX * 1024u;
+  // a wave's 32 x 32 tiles: 2 of rows x 2 of tokens, or 1 x 2 where the tile has 64 tokens
+  constexpr u32 RT = NJ == 1 ? 1u : 2u, JT = 2u;
   // a ring of 2 stages (one in flight), or of 3 where 64 tokens leave the LDS and a stage is shorter than a load's
   // way from memory (the 64-token tiles; one in flight is what fits beside the 128-token ones)
   constexpr u32 NBUF = NJ == 1 ? 3u : 2u, NWAIT = (NBUF - 2u) * (NF + NA / 4u);
@@ -3192,7 +3196,7 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
   static_assert(NR >= 1u && NR <= 3u && !(Q6 && NR != 1u), "the last loads of a stage");
   __shared__ __attribute__((aligned(1024))) uint8_t sm_[GR * GL > OB ? GR * GL : OB];
   const u32 tid = threadIdx.x, lane = tid & 63u, w = __builtin_amdgcn_readfirstlane(tid >> 6) & (4u * GR - 1u);
-  const u32 grp = GR == 2 ? w >> 2 : 0u, wq = w & 3u, wm = w & 1u, wn = (w >> 1) & 1u, l32 = lane & 31u, kg = lane >> 5;
+  const u32 grp = GR == 2 ? w >> 2 : 0u, wq = w & 3u, wm = RT == 1u ? wq : w & 1u, wn = RT == 1u ? 0u : (w >> 1) & 1u, l32 = lane & 31u, kg = lane >> 5;
   const u32 ng = amdc_ngroups(nb);
   const u32 ntt = (T + TW - 1u) / TW, b = blockIdx.x, full = b < nfull;
   const u32 tail = (rows + 127u) / 128u * ntt - nfull, tj = b - nfull;
@@ -3274,11 +3278,11 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
     }
   };
 
-  v16f acc[2][NJ], tmp[PB ? 1 : 2][NJ];
+  v16f acc[RT][JT], tmp[PB ? 1 : RT][JT];
 #pragma unroll
-  for (u32 i = 0; i < 2u; i++)
+  for (u32 i = 0; i < RT; i++)
 #pragma unroll
-    for (u32 j = 0; j < (u32)NJ; j++) acc[i][j] = (v16f)(0.0f), tmp[PB ? 0u : i][j] = (v16f)(0.0f);
+    for (u32 j = 0; j < JT; j++) acc[i][j] = (v16f)(0.0f), tmp[PB ? 0u : i][j] = (v16f)(0.0f);
   const KW kc = kw();
   // the first super-group's headers and tables
   u32 g = g0 + grp, par = 0u, slot = 0u;
@@ -3291,8 +3295,8 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
   build(g, 64u, 0u);
   if (GR == 2 && grp) __builtin_amdgcn_s_barrier(); // the second group runs half a stage behind the first
   // lane offsets inside a stage
-  const u32 rl = 64u * wm + l32;
-  const u32 la = OA + rl * 16u + (Q8 ? 2048u * kg : 8u * kg), lb = 2u * NJ * wn * 1024u + 16u * lane, ld = 128u * TW + 4u * (32u * NJ * wn + l32);
+  const u32 rl = 32u * RT * wm + l32;
+  const u32 la = OA + rl * 16u + (Q8 ? 2048u * kg : 8u * kg), lb = 2u * JT * wn * 1024u + 16u * lane, ld = 128u * TW + 4u * (32u * JT * wn + l32);
   const u32 lx = 128u * TW + 1024u + (NJ == 2 ? 1024u * wn : 0u) + 16u * lane;
   // the A operands of block bb of stage q, row tile i (Q6_K: [s] hi, [2 + s] lo)
   constexpr u32 NFR = Q6 ? 4u : 2u;
@@ -3346,46 +3350,47 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
         if (GR == 2 && bb == 1u) __builtin_amdgcn_s_barrier(); // the other group's stage begins
         __builtin_amdgcn_sched_barrier(0);
         if (!on) continue;
-        h8 bf[NJ][2], af[Q6 ? 1 : 2][NFR]; // Q6_K: one row tile's operands at a time (registers)
+        h8 bf[JT][2], af[Q6 ? 1 : RT][NFR]; // Q6_K: one row tile's operands at a time (registers)
 #pragma unroll
-        for (u32 i = 0; i < (Q6 ? 1u : 2u); i++) frag(base, tb, q, bb, i, af[i]);
+        for (u32 i = 0; i < (Q6 ? 1u : RT); i++) frag(base, tb, q, bb, i, af[i]);
 #pragma unroll
-        for (u32 j = 0; j < (u32)NJ; j++)
+        for (u32 j = 0; j < JT; j++)
 #pragma unroll
           for (u32 s = 0; s < 2u; s++) bf[j][s] = *(const h8 *)(base + lb + 64u * TW * bb + (2u * j + s) * 1024u);
         if constexpr (PB) {
           // d_w d_a of the tile's rows and tokens as an outer product on the matrix unit (rank 1, one rounding), row tiles 0
-          // and 1 in its two blocks; then acc += (d_w d_a) X per element
-          const float dw = *(const float *)(tb + ((2u * q + bb) * 128u + rl + 32u * kg) * 4u);
-          v32f pr[NJ];
+          // and 1 (one row tile: token tiles 0 and 1) in its two blocks; then acc += (d_w d_a) X per element
+          const float dw = *(const float *)(tb + ((2u * q + bb) * 128u + rl + (RT == 2u ? 32u * kg : 0u)) * 4u);
+          v32f pr[RT];
 #pragma unroll
-          for (u32 j = 0; j < (u32)NJ; j++) {
-            const float dj = *(const float *)(base + ld + 4u * TW * bb + 128u * j);
+          for (u32 j = 0; j < RT; j++) {
+            const float dj = *(const float *)(base + ld + 4u * TW * bb + 128u * (RT == 2u ? j : kg));
             pr[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dj, (v32f)(0.0f), 0, 0, 0);
           }
           v16f x[2];
           x[0] = mma(af[0], bf[0]);
 #pragma unroll
-          for (u32 t = 0; t < 2u * NJ; t++) {
-            if (t + 1u < 2u * NJ) x[(t + 1u) & 1u] = mma(af[(t + 1u) / NJ], bf[(t + 1u) % NJ]);
-            const u32 i = t / NJ, j = t % NJ;
+          for (u32 t = 0; t < RT * JT; t++) {
+            if (t + 1u < RT * JT) x[(t + 1u) & 1u] = mma(af[(t + 1u) / JT], bf[(t + 1u) % JT]);
+            const u32 i = t / JT, j = t % JT;
 #pragma unroll
-            for (u32 v = 0; v < 16u; v++) acc[i][j][v] = __builtin_fmaf(pr[j][16u * i + v], x[t & 1u][v], acc[i][j][v]);
+            for (u32 v = 0; v < 16u; v++)
+              acc[i][j][v] = __builtin_fmaf(RT == 2u ? pr[j % RT][16u * i + v] : pr[0][16u * j + v], x[t & 1u][v], acc[i][j][v]);
           }
         } else {
-          float dj[NJ];
+          float dj[JT];
 #pragma unroll
-          for (u32 j = 0; j < (u32)NJ; j++) dj[j] = *(const float *)(base + ld + 4u * TW * bb + 128u * j);
+          for (u32 j = 0; j < JT; j++) dj[j] = *(const float *)(base + ld + 4u * TW * bb + 128u * j);
           v16f x[2];
           x[0] = mma(af[0], bf[0]);
 #pragma unroll
-          for (u32 t = 0; t < 2u * NJ; t++) {
-            if (Q6 && t + 1u == (u32)NJ) {
+          for (u32 t = 0; t < RT * JT; t++) {
+            if (Q6 && RT == 2u && t + 1u == JT) {
               __builtin_amdgcn_sched_barrier(0);
               frag(base, tb, q, bb, 1u, af[0]);
             }
-            if (t + 1u < 2u * NJ) x[(t + 1u) & 1u] = mma(af[Q6 ? 0u : (t + 1u) / NJ], bf[(t + 1u) % NJ]);
-            const u32 i = t / NJ, j = t % NJ;
+            if (t + 1u < RT * JT) x[(t + 1u) & 1u] = mma(af[Q6 ? 0u : (t + 1u) / JT], bf[(t + 1u) % JT]);
+            const u32 i = t / JT, j = t % JT;
 #pragma unroll
             for (u32 v = 0; v < 16u; v++)
               tmp[i][j][v] = q == 0u && bb == 0u ? dj[j] * x[t & 1u][v] : __builtin_fmaf(dj[j], x[t & 1u][v], tmp[i][j][v]);
@@ -3394,13 +3399,13 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
       }
       __builtin_amdgcn_sched_barrier(0);
       if (!PB && on) {
-        // Q4_K: the min term of one of the wave's token groups: - (dmin mn) (d_a asum) over the super-group's 8 blocks,
+        // Q4_K: the min term of one of the wave's two token groups: - (dmin mn) (d_a asum) over the super-group's 8 blocks,
         // m1 x1 + m1 x2 + m2 x1 + m2 x2 + m1 x3 + m2 x3
-        if (Q4K && (NJ == 2 || wn == (q >> 1))) {
-          const u32 j = NJ == 2 ? q >> 1 : 0u;
+        if (Q4K) {
+          const u32 j = q >> 1;
           const b8 xb = *(const b8 *)(base + lx);
 #pragma unroll
-          for (u32 i = 0; i < 2u; i++) {
+          for (u32 i = 0; i < RT; i++) {
             const uint8_t *l = tb + 4096u + (rl + 32u * i) * 16u;
             if ((q & 1u) == 0u) {
               acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const b8 *)l, xb, acc[i][j], 0, 0, 0);
@@ -3412,14 +3417,14 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
         }
         if (q == 3u) { // the end of the super-block: d of the C rows 8 (v / 4) + 4 kg + v % 4
 #pragma unroll
-          for (u32 i = 0; i < 2u; i++)
+          for (u32 i = 0; i < RT; i++)
 #pragma unroll
             for (u32 v4 = 0; v4 < 4u; v4++) {
-              const v4f dv = *(const v4f *)(tb + 8192u + (64u * wm + 32u * i + 8u * v4 + 4u * kg) * 4u);
+              const v4f dv = *(const v4f *)(tb + 8192u + (32u * RT * wm + 32u * i + 8u * v4 + 4u * kg) * 4u);
 #pragma unroll
               for (u32 v = 0; v < 4u; v++)
 #pragma unroll
-                for (u32 j = 0; j < (u32)NJ; j++)
+                for (u32 j = 0; j < JT; j++)
                   acc[i][j][4u * v4 + v] = __builtin_fmaf(dv[v], tmp[PB ? 0u : i][j][4u * v4 + v], acc[i][j][4u * v4 + v]);
             }
         }
@@ -3438,12 +3443,12 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
   for (u32 ph = 0; ph < (u32)GR; ph++) {
     if (GR == 1 || grp != ph) {
 #pragma unroll
-      for (u32 i = 0; i < 2u; i++)
+      for (u32 i = 0; i < RT; i++)
 #pragma unroll
-        for (u32 j = 0; j < (u32)NJ; j++)
+        for (u32 j = 0; j < JT; j++)
 #pragma unroll
           for (u32 v4 = 0; v4 < 4u; v4++) {
-            v4f *o = (v4f *)&so[(32u * (NJ * wn + j) + l32) * OSTR + 64u * wm + 32u * i + 8u * v4 + 4u * kg];
+            v4f *o = (v4f *)&so[(32u * (JT * wn + j) + l32) * OSTR + 32u * RT * wm + 32u * i + 8u * v4 + 4u * kg];
             v4f a = {acc[i][j][4u * v4], acc[i][j][4u * v4 + 1u], acc[i][j][4u * v4 + 2u], acc[i][j][4u * v4 + 3u]};
             if (ph == 1u) a = a + *o;
             *o = a;
