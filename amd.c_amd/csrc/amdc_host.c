@@ -220,6 +220,7 @@ static struct {
   hipError_t (*StreamDestroy)(hipStream_t);
   hipError_t (*StreamSynchronize)(hipStream_t);
   hipError_t (*StreamWaitEvent)(hipStream_t, hipEvent_t, unsigned);
+  hipError_t (*StreamIsCapturing)(hipStream_t, int *);
   hipError_t (*StreamBeginCapture)(hipStream_t, int);
   hipError_t (*StreamEndCapture)(hipStream_t, hipGraph_t *);
   hipError_t (*GraphInstantiate)(hipGraphExec_t *, hipGraph_t, void *, char *, size_t);
@@ -402,6 +403,7 @@ static int hip_load(void) {
   SYM(StreamDestroy, "hipStreamDestroy");
   SYM(StreamSynchronize, "hipStreamSynchronize");
   SYM(StreamWaitEvent, "hipStreamWaitEvent");
+  SYM(StreamIsCapturing, "hipStreamIsCapturing");
   SYM(StreamBeginCapture, "hipStreamBeginCapture");
   SYM(StreamEndCapture, "hipStreamEndCapture");
   SYM(GraphInstantiate, "hipGraphInstantiate");
@@ -759,6 +761,10 @@ static u32 gemv2_lanes(u32 ng, u32 rows, int k8) {
 #define GEMV_LDS_T1 (150u * 1024u)
 
 static int ws_take(size_t n, void **p);
+/* Whether n bytes of workspace are there, or can be allocated: not while the stream is captured. The Q6_K
+ * choices that need a workspace where others do not (a K split of at most 4 tiles, the verify kernel in place of
+ * amdc_gemv_q6_k_m1) ask it, so that those calls can always be captured. */
+static int ws_ready(size_t n, void *stream);
 
 /* The verify GEMV on int8 MFMA (T <= 16): 64 rows per workgroup, K split
  * over aligned ranges of tiles (64 blocks each): for T <= 8 until the
@@ -821,6 +827,7 @@ static int gemv8_launch(int kind, const void *w, const uint8_t *xq, float *y, ui
       const double r = (double)wgs * n / slots, est = (r > 1.0 ? r : 1.0) * (S < nt ? S : nt) + (n > 1u ? 1.0 : 0.0);
       if (est <= best) best = est, tps = S;
     }
+    if (nt <= 4u && !ws_ready((size_t)((nt + tps - 1u) / tps) * T * rows * 4u, stream)) tps = 4u;
   }
   const u32 ks = (nt + tps - 1u) / tps;
   float *part = NULL;
@@ -989,7 +996,7 @@ static int gemv_launch(int kind, const void *w, const uint8_t *xq, float *y, uin
          17.6; 17408 x 5120 T = 2 25.1 / 28.7: Q6_K past T = 2 counts its idle lanes too. Q8_0 4096 x 4096 6.4 / 9.5, 7.8 / 9.6, 10.6 / 10.1; 11008 x 4096 T = 2, 4 12.3 /
          15.2, 15.4 / 14.9; 1024 x 2048 T = 8 7.6 / 6.5: Q8_0 only up to T = 4 and half the size */
       const u64 lim = kind == AMDC_KIND_Q6_K ? M8_MAX : T <= 4u ? M8_MAX * 2u / 3u : 0u;
-      const u32 gl = kind == AMDC_KIND_Q6_K && T > 2u ? L : ng;
+      const u32 gl = kind == AMDC_KIND_Q6_K && T > 2u && ws_ready((size_t)16u * T * rows * 4u, stream) ? L : ng;
       if (ni == 1u && lds <= 64u * 1024u && (u64)T * rows * gl <= lim && (u64)rows * rb + rb < (1ull << 32)) {
         void *a[] = {&w, &xq, &y, &rows, &nb, &bias, &res, (void *)&L, &T, &xs, &ys, &rs};
         return launch(K_GEMVM8 + (kind == AMDC_KIND_Q6_K ? 1 : 0), nrg, 1, lds, stream, a);
@@ -1292,6 +1299,12 @@ static int ws_reserve(size_t n) {
   HIPCALL(H.Malloc(&g_ws, m));
   g_ws_bytes = m;
   return AMDC_OK;
+}
+
+static int ws_ready(size_t n, void *stream) {
+  int st = 0; /* hipStreamCaptureStatusNone */
+  if (n <= (g_ws_fixed ? g_scratch_bytes : g_ws_bytes)) return 1;
+  return !g_ws_fixed && (!stream || (H.StreamIsCapturing(stream, &st) == 0 && st == 0));
 }
 
 /* The workspace of an operator: n bytes at *p, from the grown allocation, or from the fixed

@@ -1,6 +1,9 @@
 """The Q6_K verify GEMV (amdc_gemv_q6_k_v8 / _v16) on an MI355X: every token's bits are the decode GEMV's, at the edges of
 its row groups, tiles, ranges and token halves, on ordinary weights and on the extremes of the format (weights -32 and
 31 on scales -128 and 127 with activations of -127 and 127: the largest half dots)."""
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -51,3 +54,32 @@ def test_bits_of_decode(dev, rows, nb, ks, T, extreme):
         assert np.array_equal(Y.download(np.uint32)[:T * rows].reshape(T, rows), np.stack(want))
     finally:
         dev.set_tuning()
+
+
+@pytest.mark.parametrize("rows,nb,T", [(4096, 128, 16), (3200, 344, 4)])
+def test_first_call_under_capture(rows, nb, T):
+    """In a fresh process, whose workspace holds nothing yet: a captured call replays with the eager call's bits."""
+    code = f"""
+import sys; sys.path[:0] = {sys.path!r}
+import numpy as np, amdc as dev
+from amdc import synth
+dev.open_device()
+rows, nb, T = {rows}, {nb}, {T}
+xs = (40 * nb + 255) // 256 * 256
+g = np.random.default_rng(1)
+W = dev.DevBuf.of(np.resize(dev.repack(4, synth.gguf(4, 40, 32 * nb, 1), 40, 32 * nb), dev.mat_bytes(4, rows, 32 * nb)))
+X, Q, Y = dev.DevBuf.of(synth.activations(T, 32 * nb, 2)), dev.DevBuf(T * xs), dev.DevBuf(4 * T * rows)
+Q.fill(0)
+dev.quant_q8(X, Q, nb, T, 128 * nb, xs)
+S = dev.Stream()
+S.sync()
+G = dev.Graph(S, lambda s: dev.gemv_t(4, W, Q, Y, rows, nb, T, xs, rows, stream=s))
+out = []
+for rep in range(3):
+    Y.fill(0xEE); G.launch(); S.sync(); out.append(Y.download(np.uint32))
+    Y.fill(0xEE); dev.gemv_t(4, W, Q, Y, rows, nb, T, xs, rows); out.append(Y.download(np.uint32))
+assert all(np.array_equal(o, out[0]) for o in out)
+print("same")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "same" in r.stdout, r.stderr[-800:]
