@@ -5,13 +5,13 @@
 // kernels (hanw/amd.c src/hip.c:102-107, 568-598).
 //
 // Kernels (grid x = workgroups, 256 threads each):
-//   amdc_quant_q8      Q8 activation quantization (src/cpu.c:36-53)
-//   amdc_rmsnorm_q8, amdc_swiglu_q8
-//                      the Q8 producers (the float op and its Q8 copy)
+//   amdc_quant_q8, _v  Q8 activation quantization (src/cpu.c:36-53; _v: aligned rows)
+//   amdc_rmsnorm_q8, _r, amdc_swiglu_q8, _v
+//                      the Q8 producers (the float op and its Q8 copy; _r, _v: aligned rows)
 //   amdc_gemv_{q4_0,q4_k}_p1, _x1, {q4_0,q4_k,q8_0,q6_k}_p2
 //                      the decode GEMV (T = 1): short rows (_p1; _x1 with the
-//                      quantization fused), long rows and the Q8_0 / Q6_K kinds
-//                      (_p2) (ie_gemv_q4q8, ie_gemv_q4kq8, ie_gemv_q8q8,
+//                      quantization fused), long rows (_p2); amdc_gemv_{q8_0,q6_k}_s1, _xs1,
+//                      q8_0_s2, _xs2 the Q8_0 / Q6_K single-shot forms (ie_gemv_q4q8, ie_gemv_q4kq8, ie_gemv_q8q8,
 //                      ie_gemv_q6kq8)
 //   amdc_gemv_{q4_0,q4_k,q8_0,q6_k}_v8, amdc_gemv_{q4_0,q4_k,q8_0,q6_k}_v16,
 //   amdc_gemm_reduce   the verify GEMV, T <= 8 (_v8) or 16 (_v16) vectors on
