@@ -3015,9 +3015,11 @@ __device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t rs, __attribut
 
 // ------------------------------------------------------------------ prefill GEMM, wide wave tiles
 
+typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 
 // The image of the activations that amdc_gemmw_* loads straight into the LDS, 1 KB at a time: token tiles
 // of TW (64 or 128) tokens, per tile 4 ceil(nb / 8) stages of two blocks (2q, 2q + 1 of super-group g, in
@@ -3025,8 +3027,8 @@ typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 //   B operands  2 blocks x TW / 32 token groups x 2 steps x 64 lanes x 16 bytes: lane (token t % 32, half h =
 //               lane / 32) of step s holds 8 activations as f16, in the order of the weights' A operand
 //   d_a         2 blocks x TW f32 (padded to 1 KB)
-//   Q4_K only: d_a asum of the super-group's 8 blocks as three bf16 parts x = x1 + x2 + x3 (exact), for
-//               the min term: TW / 64 of the tile's TW / 16 chunks of 1 KB, chunk (token group, F): lane
+//   Q4_K only: d_a asum of the super-group's 8 blocks as three bf16 parts x = x1 + x2 + x3 (exact from
+//               2^-110 up), for the min term: TW / 64 of the tile's TW / 16 chunks of 1 KB, chunk (token group, F): lane
 //               (token, h): F = 0: h ? x2 : x1, F = 1: x3 (8 bf16, the 8 blocks). Tiles of 64: stage
 //               q holds chunk (q / 2, q % 2); tiles of 128: stage q holds chunks (q / 2, q % 2) and
 //               (2 + q / 2, q % 2), one for each half of the waves
@@ -3094,11 +3096,16 @@ extern "C" __global__ __launch_bounds__(256) void amdc_gemmw_prep(const uint8_t 
 #pragma unroll
     for (u32 b = 0; b < 8u; b++) {
       const float x = sx[b][tl];
-      const u32 x1 = __builtin_bit_cast(u32, x) & 0xFFFF0000u;
-      const float r1 = x - __builtin_bit_cast(float, x1);
-      const u32 x2 = __builtin_bit_cast(u32, r1) & 0xFFFF0000u;
-      const u32 x3 = __builtin_bit_cast(u32, r1 - __builtin_bit_cast(float, x2));
-      part[b] = w ? x3 : h ? x2 : x1;
+      float x1 = __builtin_bit_cast(float, __builtin_bit_cast(u32, x) & 0xFFFF0000u), r1 = x - x1;
+      float x2 = __builtin_bit_cast(float, __builtin_bit_cast(u32, r1) & 0xFFFF0000u), x3 = r1 - x2;
+      // no part of an x other than 0 is 0 (a part that is gets a share of the one before, exact): the product of
+      // an infinite min with a zero part would be a NaN
+      if (r1 == 0.0f) x3 = x2 = 0.25f * x1, x1 = 0.5f * x1;
+      else if (x3 == 0.0f) x3 = x2 = 0.5f * x2;
+      // an infinite or NaN x is the part that only the min's first part meets (lanes of half 0 of chunk F = 1)
+      if (!__builtin_isfinite(x)) x1 = x2 = __builtin_copysignf(1.0f, x), x3 = h ? 0.0f : x;
+      part[b] = __builtin_bit_cast(u32, w ? x3 : h ? x2 : x1);
+      if (x != x) part[b] |= 0x00400000u; // (quiet: the 16 bits kept are a NaN's)
     }
     u32x4 o;
 #pragma unroll
@@ -3240,7 +3247,7 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
   };
   // the tables of 64 rows (rb ..) of super-group g from their headers: thread (row, blocks 2 wq, 2 wq + 1):
   //   Q4_K: sc [block pair][row] x 2 blocks: f16 (sc, sc / 16); at 4096 min [2][row]: - dmin mn of the 8 blocks as
-  //         two bf16 parts (at most 17 bits: the part rounded to nearest leaves at most 8); at 8192 d [row] f32
+  //         two bf16 parts (at most 17 bits: the part rounded to nearest leaves at most 8, below 2^14); at 8192 d [row] f32
   //   Q6_K: sc [block pair][row] x 2 blocks x 2 halves: f16 (sc >> 4, (sc & 15) / 16); at 8192 16 d [row] f32
   //   Q4_0, Q8_0: d [block][row] f32
   auto build = [&](u32 g, u32 rb, u32 par) {
@@ -3269,10 +3276,11 @@ __device__ __forceinline__ void gemmw_body(const uint8_t *__restrict__ W, const 
       const u32 a = __builtin_bit_cast(u32, sc), c = __builtin_bit_cast(u32, sd);
       *(u32x2 *)(t + (wq * 128u + r) * 8u) = (u32x2){__builtin_amdgcn_perm(c, a, 0x05040100u), __builtin_amdgcn_perm(c, a, 0x07060302u)};
       const float dm = -h2f(h.x >> 16), m0 = dm * (float)(n2 & 63u), m1 = dm * (float)((n2 >> 6) & 63u);
-      const u32 p0 = __builtin_bit_cast(u32, m0) + 0x8000u, p1 = __builtin_bit_cast(u32, m1) + 0x8000u;
-      const float q0 = m0 - __builtin_bit_cast(float, p0 & 0xFFFF0000u), q1 = m1 - __builtin_bit_cast(float, p1 & 0xFFFF0000u);
+      const u32 p = __builtin_bit_cast(u32, __builtin_convertvector((v2f){m0, m1}, b2));
+      // (the maximum: an infinite min is its first part alone, beside a finite second one)
+      const float q0 = __builtin_fmaxf(m0 - __builtin_bit_cast(float, p << 16), -16384.0f), q1 = __builtin_fmaxf(m1 - __builtin_bit_cast(float, p & 0xFFFF0000u), -16384.0f);
       u32 *l = (u32 *)(t + 4096u + r * 16u + 4u * wq);
-      l[0] = __builtin_amdgcn_perm(p1, p0, 0x07060302u);
+      l[0] = p;
       l[512] = __builtin_amdgcn_perm(__builtin_bit_cast(u32, q1), __builtin_bit_cast(u32, q0), 0x07060302u);
       if (wq == 0u) *(float *)(t + 8192u + r * 4u) = h2f(h.x);
     }

@@ -81,3 +81,87 @@ def test_noalloc_falls_back(dev, orc):
     y = c.y_gpu()
     for t in range(0, T, 111):
         assert rel_err(y[t], c.y_oracle(t), c.mag(t)) < TOL, t
+
+
+# ---------------------------------------------------------------- infinities, NaN, zeros
+
+D_OFF = {synth.KIND_Q4_0: (18, 0), synth.KIND_Q8_0: (34, 0), synth.KIND_Q4_K: (144, 0), synth.KIND_Q6_K: (210, 208)}  # block bytes, its d
+
+
+def special_weights(kind, rows, nb, seed):
+    """(bytes, rows with a special scale): infinite and NaN d, Q4_K: dmin, in one block of a row each; Q4_K: a row
+    whose sub-block scales are all 0 (its products are 0 beside an infinite min term)."""
+    size, off = D_OFF[kind]
+    src = synth.gguf(kind, rows, 32 * nb, seed).reshape(rows, -1).copy()
+    n = src.shape[1] // size
+    f16 = np.array([np.inf, -np.inf, np.nan], np.float16).view(np.uint8).reshape(3, 2)
+    for i in range(3):
+        o = min(i, n - 1) * size + off
+        src[5 + i, o:o + 2] = f16[i]
+        if kind == synth.KIND_Q4_K:
+            src[9 + i, o + 2:o + 4] = f16[i]
+    if kind == synth.KIND_Q4_K:
+        for g in range(n):  # sc 0..3 = 0, mn 0..3 kept; sc 4..7 = 0, mn 4..7 their low 4 bits
+            h = src[20, g * size + 4:g * size + 16]
+            h[0:4], h[4:8], h[8:12] = 0, h[4:8] & 63, h[8:12] & 0xF0
+    return src.reshape(-1), list(range(5, 12)) + [20]
+
+
+def special_tokens(xq, nb):
+    """Tokens 3 .. 12 of the Q8 rows xq get special blocks; their numbers."""
+    q = xq[:, :32 * nb].view(np.int8)
+    d = xq[:, 32 * nb:36 * nb].view(np.float32)
+    a = xq[:, 36 * nb:40 * nb].view(np.int32)
+
+    def block(t, b, val, dd):
+        q[t, 32 * b:32 * b + 32], d[t, b], a[t, b] = val, dd, 32 * val
+
+    d[3, 4], d[4, 1], d[5, 9] = np.inf, -np.inf, np.nan
+    for b in range(nb):
+        block(6, b, 0, 0.0)     # the zero token
+        block(9, b, 2, 1.0)     # d_a asum = 64: one significant bit
+        block(10, b, b % 3, 1.0)  # some blocks 0 under every min
+        block(12, b, 1, 1e-20)
+    block(7, 2, 127, 1e37)      # d_a asum overflows to an infinity of each sign
+    block(8, 3, -127, 1e37)
+    block(11, 0, 127, 1e28)     # large and finite
+    return list(range(3, 13))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("T,ks", [(40, 0), (70, 0), (150, 0), (150, 2)])
+def test_special_values(dev, orc, kind, T, ks):
+    """Infinite, NaN and zero blocks in activations and weights: infinities of the same sign and NaN at the same
+    places as from the 64-row kernels, whose min term is in f32; the other rows and tokens keep their bits."""
+    rows, nb = 140, 24
+    src, srows = special_weights(kind, rows, nb, seed=kind + T)
+    xq = orc.quant_q8(synth.activations(T, 32 * nb, kind + T)).reshape(T, 40 * nb).copy()
+    clean_src, clean_xq = synth.gguf(kind, rows, 32 * nb, kind + T), xq.copy()
+    stok = special_tokens(xq, nb)
+    xs = (40 * nb + 255) // 256 * 256
+
+    def run(s, x, kern):
+        pad = np.zeros((T, xs), np.uint8)
+        pad[:, :40 * nb] = x
+        W, Q, Y = dev.DevBuf.of(dev.repack(kind, s, rows, 32 * nb)), dev.DevBuf.of(pad), dev.DevBuf(4 * T * rows)
+        Y.fill(0x55)
+        dev.set_tuning(gemm_kernel=kern, gemm_ksplit=ks)
+        try:
+            dev.gemm(kind, W, Q, Y, rows, nb, T, xs, rows)
+        finally:
+            dev.set_tuning()
+        return Y.download(np.float32).reshape(T, rows)
+
+    want, got, clean = run(src, xq, 4), run(src, xq, 5), run(clean_src, clean_xq, 5)
+    for cls in (np.isnan, np.isposinf, np.isneginf):
+        bad = np.argwhere(cls(got) != cls(want))
+        assert len(bad) == 0, (cls.__name__, len(bad), bad[:5].tolist(), [(float(got[t, r]), float(want[t, r])) for t, r in bad[:5]])
+    rest = [r for r in range(rows) if r not in srows]
+    other = [t for t in range(T) if t not in stok]
+    assert np.array_equal(got[np.ix_(other, rest)].view(np.uint32), clean[np.ix_(other, rest)].view(np.uint32))
+    for t in stok:
+        if t in (6, 9, 10, 12):
+            mag = orc.gemv_f64(synth.GGML[kind], src, rows, nb, xq[t])[1][rest]
+            assert rel_err(got[t, rest], want[t, rest], mag) < TOL, t
+    assert np.isinf(want).any() and np.isnan(want).any() and np.all(got[6, rest] == 0.0)
