@@ -1377,37 +1377,61 @@ static gw_plan gw_choose(int kind, u32 rows, u32 ng, u32 T, u32 cus) {
   return best;
 }
 
-static int gemmw_launch(int kind, const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias,
-                        const float *res, uint32_t T, uint32_t xs, uint32_t ys, uint32_t rs, void *stream) {
-  const u32 ng = amdc_ngroups(nb), cus = g_cus > 0 ? (u32)g_cus : 256u;
-  gw_plan p = gw_choose(kind, rows, ng, T, cus);
-  if (t_ksplit > 0) p.form = T <= 64u ? GW_J64 : GW_J128;
-  const u32 TW = p.form == GW_J64 ? 64u : 128u, ind = p.form == GW_I128;
-  const u32 ntt = (T + TW - 1u) / TW, tiles = (rows + 127u) / 128u * ntt;
-  if (t_ksplit > 0) {
-    const u32 np = ind ? ng : (ng + 1u) / 2u;
-    p.ks = (u32)t_ksplit < np ? (u32)t_ksplit : np, p.nfull = p.ks > 1u ? 0u : tiles; /* (unsplit tiles go to y) */
-  }
+/* The image of a token tile (amdc_gemmw_prep: 4 ng stages), and the partial sums of nt tokens and nr rows */
+static size_t gw_image(int kind, u32 form, u32 ng) {
+  const size_t tw = form == GW_J64 ? 64u : 128u;
+  return (size_t)ng * 4u * (128u * tw + 1024u + (kind == AMDC_KIND_Q4_K ? 16u * tw : 0u));
+}
+static size_t gw_part(u32 ks, u32 nt, u32 nr) { return ks > 1u ? (size_t)ks * nt * nr * 4u : 0u; }
+
+/* rows x T outputs by plan p (its tiles [0, nfull) counted in these rows and tokens) */
+static int gemmw_run(int kind, gw_plan p, const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias,
+                     const float *res, uint32_t T, uint32_t xs, uint32_t ys, uint32_t rs, void *stream) {
+  const u32 ng = amdc_ngroups(nb), TW = p.form == GW_J64 ? 64u : 128u, ntt = (T + TW - 1u) / TW, tiles = (rows + 127u) / 128u * ntt;
   const int k = K_GEMMW + 3 * (int)gw_kind(kind) + (int)p.form;
   const u32 r0 = p.nfull / ntt * 128u, trows = rows > r0 ? rows - r0 : 0u; /* the split tail's rows */
   u32 ord = kind == AMDC_KIND_Q8_0 ? 1u : kind == AMDC_KIND_Q6_K ? 2u : 0u, q4k = kind == AMDC_KIND_Q4_K;
-  /* the image (amdc_gemmw_prep: 4 ng stages per token tile) and the partial sums */
-  const size_t img_b = (size_t)ntt * ng * 4u * (128u * TW + 1024u + (q4k ? 16u * TW : 0u)), part_b = p.ks > 1u ? (size_t)p.ks * T * trows * 4u : 0u;
+  const size_t img_b = ntt * gw_image(kind, p.form, ng);
   const u64 grid = (u64)p.nfull + (u64)(tiles - p.nfull) * p.ks;
-  if (grid > 0x7FFFFFFFull || (g_ws_fixed && img_b + part_b > g_scratch_bytes)) return -1;
   uint8_t *ws = NULL;
-  int rc = ws_take(img_b + part_b, (void **)&ws);
+  int rc = ws_take(img_b + gw_part(p.ks, T, trows), (void **)&ws);
   if (rc) return rc;
   void *img = ws, *part = p.ks > 1u ? (void *)(ws + img_b) : NULL;
   void *pa[] = {&xq, &nb, &T, &xs, &img, (void *)&TW, &ord, &q4k};
   if ((rc = launch(K_GEMMW_PREP, (unsigned)(ng * (ntt * TW / 32u)), 1, 0, stream, pa))) return rc;
   void *ga[] = {&w, &img, &y, &rows, &nb, &bias, &res, &T, &ys, &rs, &part, &p.nfull, &p.ks};
-  if ((rc = launch_nt(k, (unsigned)grid, 1, ind ? 256u : 512u, 0, stream, ga)) || p.ks == 1u) return rc;
+  if ((rc = launch_nt(k, (unsigned)grid, 1, p.form == GW_I128 ? 256u : 512u, 0, stream, ga)) || p.ks == 1u) return rc;
   const u64 n = (u64)trows * T; /* the tail rows: y, bias and res from row r0 */
   float *yt = y + r0;
   const float *bt = bias ? bias + r0 : NULL, *rt = res ? res + r0 : NULL;
   void *ra[] = {&part, &p.ks, &yt, (void *)&trows, &T, &bt, &rt, &ys, &rs};
   return launch(K_GEMM_REDUCE, (unsigned)((n + 255u) / 256u), 1, 0, stream, ra);
+}
+
+static int gemmw_launch(int kind, const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias,
+                        const float *res, uint32_t T, uint32_t xs, uint32_t ys, uint32_t rs, void *stream) {
+  const u32 ng = amdc_ngroups(nb), cus = g_cus > 0 ? (u32)g_cus : 256u;
+  gw_plan p = gw_choose(kind, rows, ng, T, cus);
+  if (t_ksplit > 0) p.form = T <= 64u ? GW_J64 : GW_J128;
+  const u32 TW = p.form == GW_J64 ? 64u : 128u, ntt = (T + TW - 1u) / TW, tiles = (rows + 127u) / 128u * ntt;
+  if (t_ksplit > 0) p.ks = (u32)t_ksplit < (ng + 1u) / 2u ? (u32)t_ksplit : (ng + 1u) / 2u, p.nfull = p.ks > 1u ? 0u : tiles; /* (unsplit tiles go to y) */
+  if ((u64)p.nfull + (u64)(tiles - p.nfull) * p.ks > 0x7FFFFFFFull) return -1;
+  const u32 rt = p.nfull / ntt, trows = p.ks > 1u ? rows - rt * 128u : 0u; /* row tiles over the whole K; rows in splits */
+  const size_t img = gw_image(kind, p.form, ng);
+  u32 n = ntt;
+  /* Where the fixed workspace does not hold it: the same plan in pieces of n token tiles. An output's sum depends on the
+     form and its row's splits alone, so the bits are those of one piece. One token tile fits: an image of at most 20 MB
+     (2048 blocks) and partial sums of at most 2 rounds of workgroups, 64 KB each. Refused (by ws_take) where the 64-row kernels'
+     activations, 72 bytes per block and token, would not fit either. */
+  if (g_ws_fixed && (size_t)((T + 127u) / 128u) * 128u * nb * 72u <= g_scratch_bytes)
+    while (n > 1u && n * img + gw_part(p.ks, n < ntt ? n * TW : T, trows) > g_scratch_bytes) n--;
+  for (u32 t = 0; t < T; t += n * TW) {
+    const u32 Tn = T - t < n * TW ? T - t : n * TW, nt = (Tn + TW - 1u) / TW;
+    const gw_plan q = {p.form, rt * nt, p.ks};
+    const int rc = gemmw_run(kind, q, w, xq + (size_t)t * xs, y + (size_t)t * ys, rows, nb, bias, res ? res + (size_t)t * rs : NULL, Tn, xs, ys, rs, stream);
+    if (rc) return rc;
+  }
+  return AMDC_OK;
 }
 
 /* The prefill GEMM on the f16-MFMA kernels (every kind). */
@@ -1429,8 +1453,7 @@ static int gemm_launch(int kind, const char *op, const void *w, const uint8_t *x
   /* the wide-tile kernels, above 2^22 weights times token tiles of 64: below that the 64-row kernels' shorter way to the
      first product wins (MI355X, us, 64-row / wide: 1000 x 4096 Q4_K T = 33 13.6 / 16.9, 2048 x 2048 Q6_K T = 64
      16.1 / 19.5, 4096 x 1024 Q8_0 T = 20 12.8 / 14.9; above, 2048 x 4096 Q4_0 T = 33 18.4 / 16.2, 1000 x 8192 Q4_K T = 64
-     19.7 / 19.8, 4096 x 4096 Q4_K T = 33 27.3 / 19.0). Where the wide kernels' image and partial sums do not fit the
-     fixed workspace of amdc_op_gemv_noalloc, the 64-row ones, which need a little less */
+     19.7 / 19.8, 4096 x 4096 Q4_K T = 33 27.3 / 19.0) */
   const int small = (u64)rows * nb * 32u * ((T + 63u) / 64u) <= (1ull << 22);
   if (t_gemm == 5 || (t_gemm == 0 && !small)) {
     if ((rc = gemmw_launch(kind, w, xq, y, rows, nb, bias, res, T, xs, ys, rs, stream)) != -1) return rc;
@@ -1468,8 +1491,10 @@ static int gemm_launch(int kind, const char *op, const void *w, const uint8_t *x
   if (ks > ng) ks = ng;
   if (ks > 16u) ks = 16u; /* amdc_gemm_reduce adds at most 16 splits */
   const u32 Tp = (T + 127u) / 128u * 128u, K = 32u * nb;
-  /* the fixed workspace: as many splits as their partial sums leave room for */
-  while (g_ws_fixed && ks > 1u && (size_t)Tp * nb * 72u + (size_t)ks * T * (rows - nfull / ntt * gh[v].mr) * 4u > g_scratch_bytes) ks--;
+  /* where the activations fit the fixed workspace, as many splits as their partial sums leave room for in it (in
+     amdc_op_gemv too: the same bits) */
+  const size_t act = (size_t)Tp * nb * 72u;
+  while (ks > 1u && act <= AMDC_SCRATCH_BYTES && act + (size_t)ks * T * (rows - nfull / ntt * gh[v].mr) * 4u > AMDC_SCRATCH_BYTES) ks--;
   if (ks == 1u) nfull = tiles;
   const u32 r0 = nfull / ntt * gh[v].mr, trows = rows - r0; /* the split tail's rows */
   const size_t xh_b = (size_t)Tp * K * 2u, sc_b = (size_t)nb * Tp * 4u, part_b = ks > 1u ? (size_t)ks * T * trows * 4u : 0u;

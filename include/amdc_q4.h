@@ -253,12 +253,12 @@ int amdc_op_gemv(int kind, const void *w, const uint8_t *xq, float *y, uint32_t 
 /* amdc_op_gemv without any device allocation, for callers that cannot allocate (code under
  * HIP graph capture on a workspace size not seen before, tight serving loops, hosts that
  * forbid hipMalloc). No reference counterpart. The same kernels and launch choices as
- * amdc_op_gemv, so the same bits (a GEMM whose default kernels' workspace does not fit runs on
- * kernels and splits that need less, within the same bounds); the workspace (split-K partial sums, the GEMM's prepared
+ * amdc_op_gemv, so the same bits; the workspace (split-K partial sums, the GEMM's prepared
  * activations) is a fixed device array of AMDC_SCRATCH_BYTES in the code object, held by the
- * device from amdc_open until amdc_close. A call whose workspace would exceed it fails with
- * AMDC_EINVAL before any launch (e.g. T = 256 prefill chunks fit up to about 17408 x 5120
- * and 5120 x 17408 matrices). All calls share the one array: calls that overlap on the
+ * device from amdc_open until amdc_close. A GEMM whose workspace would exceed it runs in pieces
+ * that fit, some tokens at a time, as long as 72 bytes per block and token (T rounded up to
+ * 128) fit; another call whose workspace would exceed it fails with AMDC_EINVAL before any
+ * launch (e.g. T = 1024 with nb = 544 is refused). All calls share the one array: calls that overlap on the
  * device (other streams, graphs replayed concurrently) race; order them. Its contents are
  * whatever the last call left; no kernel needs it cleared. */
 #define AMDC_SCRATCH_BYTES ((size_t)64 << 20)

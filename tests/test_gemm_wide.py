@@ -165,3 +165,29 @@ def test_special_values(dev, orc, kind, T, ks):
             mag = orc.gemv_f64(synth.GGML[kind], src, rows, nb, xq[t])[1][rest]
             assert rel_err(got[t, rest], want[t, rest], mag) < TOL, t
     assert np.isinf(want).any() and np.isnan(want).any() and np.all(got[6, rest] == 0.0)
+
+
+@pytest.mark.gpu
+# the image alone exceeds it (Q4_K, nb = 544 and 1584: 128- and 64-token tiles), or the image and the partial sums
+# (128 tokens in two groups; two independent workgroups, whole rounds and a split tail; the longest rows)
+@pytest.mark.parametrize("kind,rows,nb,T", [(synth.KIND_Q4_K, 64, 544, 1664), (synth.KIND_Q6_K, 628, 184, 3903), (synth.KIND_Q8_0, 802, 1184, 646),
+                                            (synth.KIND_Q4_0, 15261, 552, 831), (synth.KIND_Q4_K, 290, 1584, 504), (synth.KIND_Q6_K, 1500, 2048, 380)])
+def test_noalloc_in_pieces(dev, kind, rows, nb, T):
+    """A GEMM whose workspace exceeds the fixed one gives the bits of amdc_op_gemv there too."""
+    g = np.random.default_rng(rows)
+    xs = (40 * nb + 255) // 256 * 256
+    n = dev.mat_bytes(kind, rows, 32 * nb)
+    chunk = g.integers(0, 100, min(n, 48 << 20), dtype=np.uint8)  # bytes below 100: every f16 in them is finite
+    W, Q, Y = dev.DevBuf(n), dev.DevBuf(T * xs), dev.DevBuf(4 * T * rows)
+    for o in range(0, n, len(chunk)):
+        W.upload(chunk[:min(len(chunk), n - o)], o)
+    X = dev.DevBuf.of(synth.activations(T, 32 * nb, rows))
+    R, B = dev.DevBuf.of(g.standard_normal((T, rows)).astype(np.float32)), dev.DevBuf.of(g.standard_normal(rows).astype(np.float32))
+    dev.quant_q8(X, Q, nb, T, 128 * nb, xs)
+    out = []
+    for f in (dev.op_gemv, dev.op_gemv_noalloc):
+        Y.fill(0xFF)
+        f(kind, W, Q, Y, rows, nb, T, xs, rows, rows, bias=B, res=R)
+        out.append(Y.download(np.uint32))
+    assert np.isfinite(out[0].view(np.float32)).all()
+    assert np.array_equal(out[0], out[1]), f"{int((out[0] != out[1]).sum())} of {out[0].size} outputs differ"
