@@ -288,8 +288,8 @@ enum {
   K_QUANT_V = K_GEMMW + 11, /* the producers on aligned rows: amdc_quant_q8_v, amdc_swiglu_q8_v, amdc_rmsnorm_q8_r */
   K_SWIGLU_V,
   K_RMSNORM_R,
-  K_GEMVS8, /* amdc_gemv_q8_0_s1, _s2, _xs1, _xs2, amdc_gemv_q6_k_s1, (none), _xs1 */
-  K_N = K_GEMVS8 + 7
+  K_GEMVS8, /* amdc_gemv_q8_0_s1, _s2, _xs1, (none), amdc_gemv_q6_k_s1, (none), _xs1, (none), then _s1l, _s2l, _xs1l, _xs2l, ... */
+  K_N = K_GEMVS8 + 15
 };
 #define KN(s) "amdc_" s
 #define GW(s) "amdc_gemmw_" s
@@ -318,7 +318,9 @@ static const char *const kname[K_N] = {
     GW("prep"), GW("q4_0_n128"), GW("q4_0_n64"), GW("q4_0_i128"), GW("q4_k_n128"), GW("q4_k_n64"), GW("q4_k_i128"),
     GW("q6_k_n128"), GW("q6_k_n64"), GW("q6_k_i128"), GW("q8_0_n128"), GW("q8_0_n64"),
     KN("quant_q8_v"), KN("swiglu_q8_v"), KN("rmsnorm_q8_r"),
-    KN("gemv_q8_0_s1"), KN("gemv_q8_0_s2"), KN("gemv_q8_0_xs1"), KN("gemv_q8_0_xs2"), KN("gemv_q6_k_s1"), KN("gemv_q6_k_s1"), KN("gemv_q6_k_xs1")};
+    KN("gemv_q8_0_s1"), KN("gemv_q8_0_s2"), KN("gemv_q8_0_xs1"), KN("gemv_q8_0_xs1"), KN("gemv_q6_k_s1"), KN("gemv_q6_k_s1"), KN("gemv_q6_k_xs1"),
+    KN("gemv_q6_k_xs1"), KN("gemv_q8_0_s1l"), KN("gemv_q8_0_s2l"), KN("gemv_q8_0_xs1l"), KN("gemv_q8_0_xs2l"), KN("gemv_q6_k_s1l"),
+    KN("gemv_q6_k_s1l"), KN("gemv_q6_k_xs1l")};
 
 static hipModule_t g_mod;
 static hipFunction_t g_k[K_N];
@@ -947,15 +949,15 @@ static int gemvk_launch(int kind, const void *w, const void *in, int fq, float *
 }
 
 /* The single-shot decode GEMV of the Q8_0 and Q6_K kinds (amdc_gemv_q8_0_s1 / _s2, amdc_gemv_q6_k_s1; with fq on an f32
- * vector, _xs*, quantized in every workgroup): one super-group per lane; Q8_0 also two, for rows of more than 64, and
- * with fq, as the Q4 kinds, while the grid is over 3 workgroups per CU and 8 lanes remain (22016 x 4096 16.2 us against
- * 17.8; at 4 lanes 32000 x 2048 21.2 against 12.7). -1, nothing launched, where it is not the faster form
- * (amdc_kernels.hip lists both sides): Q6_K rows of more than 64 super-groups, or on 2^16 rows and more a row that
- * leaves a quarter of its lanes idle (100000 x 5120, 20 of 32 lanes, 77.1 us against 74.6; 100000 x 4096 54.9 against
- * 58.0); Q8_0 rows of more than 128; with fq, where the workgroups quantize more than 2^17 blocks between them (us,
+ * vector, _xs*, quantized in every workgroup; _s1l and so on read the weights nontemporally): one super-group per
+ * lane; Q8_0 also two, for rows of more than 64, and with fq, while the grid is over 3 workgroups per CU, for rows that
+ * leave no lane idle (22016 x 4096 16.2 us against 17.8; 25000 x 2560, 10 super-groups, on 8 lanes 25.0, on 16 15.5). -1,
+ * nothing launched, where it is not the faster form: Q6_K rows of more than 64 super-groups; Q8_0 rows of more than 128,
+ * or of more than 64 on 4096 rows and more (us, the persistent form / this: 3000 x 17408 15.2 / 14.2, 4096 x 17408 17.9 /
+ * 17.9, 36000 x 17408 113 / 122); with fq, where the workgroups quantize more than 2^17 blocks between them (us,
  * fused / quantize launch and this form: 32000 x 4096 Q8_0 21.7 / 23.7, 32000 x 2048 Q6_K 12.3 / 14.2, 2048 x 5632 6.4 /
  * 6.9; 20000 x 5120 Q6_K 24.9 / 20.0, 60000 x 3072 33.3 / 31.1, 4096 x 11008 17.8 / 12.1); and under the tuning knobs of
- * the other forms. */
+ * the other forms. Over rows of 1000 to 36000 and 1536 to 17408 columns no launch is slower than the persistent form. */
 static int gemvs8_launch(int kind, const void *w, const void *in, int fq, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res,
                          uint8_t *q8, void *stream) {
   const u32 ng = amdc_ngroups(nb), cus = g_cus > 0 ? (u32)g_cus : 256u;
@@ -963,11 +965,16 @@ static int gemvs8_launch(int kind, const void *w, const void *in, int fq, float 
   if (t_lanes > 0 || t_wgs > 0 || (t_form != 0 && t_form != 3) || (u64)rows * rb + rb >= (1ull << 32)) return -1;
   u32 L = 4u;
   while (L < 64u && L < ng) L <<= 1;
-  if (kind == AMDC_KIND_Q6_K ? ng > 64u || (rows >= (1u << 16) && 4u * ng <= 3u * L) : ng > 128u) return -1;
-  if (fq && kind == AMDC_KIND_Q8_0 && L >= 16u && L >= ng && (rows + 4u * (64u / L) - 1u) / (4u * (64u / L)) > 3u * cus) L >>= 1;
+  if (kind == AMDC_KIND_Q6_K ? ng > 64u : ng > 128u || (ng > 64u && rows >= 4096u)) return -1;
+  if (fq && kind == AMDC_KIND_Q8_0 && L >= 16u && L == ng && (rows + 4u * (64u / L) - 1u) / (4u * (64u / L)) > 3u * cus) L >>= 1;
   const u32 ni = (ng + L - 1u) / L, rpg = 4u * (64u / L), nrg = (rows + rpg - 1u) / rpg;
   if (fq && (u64)nrg * nb > (1u << 17)) return -1;
-  const int k = K_GEMVS8 + (kind == AMDC_KIND_Q6_K ? 4 : 0) + (fq ? 2 : 0) + (int)ni - 1;
+  /* nontemporal: rows of whole 128-byte lines (load_item of these kinds), and with fq rows of more than 16 super-groups
+     where the workgroups quantize at most 2^16 blocks: there the launch is as fast either way, and the lines that it
+     leaves in L2 otherwise cost the launches after it 4 % (a step of 6144 x 2048, 2048 x 2048, 11264 x 2048, 2048 x 5632
+     and 32000 x 2048 Q8_0 40.0 us against 38.3); above, 5800 x 5120 Q6_K from L2 10.2 us nontemporally, 8.5 not */
+  const int last = rb % 128u == 0u || (fq && ng > 16u && (u64)nrg * nb <= (1u << 16));
+  const int k = K_GEMVS8 + (last ? 8 : 0) + (kind == AMDC_KIND_Q6_K ? 4 : 0) + (fq ? 2 : 0) + (int)ni - 1;
   const u32 lds = (kind == AMDC_KIND_Q6_K ? 352u : 320u) * ng;
   void *a[] = {&w, &in, &y, &rows, &nb, &bias, &res, (void *)&L, &q8};
   return launch(k, nrg, 1, lds, stream, a);

@@ -11,7 +11,7 @@
 //   amdc_gemv_{q4_0,q4_k}_p1, _x1, {q4_0,q4_k,q8_0,q6_k}_p2
 //                      the decode GEMV (T = 1): short rows (_p1; _x1 with the
 //                      quantization fused), long rows (_p2); amdc_gemv_{q8_0,q6_k}_s1, _xs1,
-//                      q8_0_s2, _xs2 the Q8_0 / Q6_K single-shot forms (ie_gemv_q4q8, ie_gemv_q4kq8, ie_gemv_q8q8,
+//                      q8_0_s2, and _s1l, .. (nontemporal loads) the Q8_0 / Q6_K single-shot forms (ie_gemv_q4q8, ie_gemv_q4kq8, ie_gemv_q8q8,
 //                      ie_gemv_q6kq8)
 //   amdc_gemv_{q4_0,q4_k,q8_0,q6_k}_v8, amdc_gemv_{q4_0,q4_k,q8_0,q6_k}_v16,
 //   amdc_gemm_reduce   the verify GEMV, T <= 8 (_v8) or 16 (_v16) vectors on
@@ -494,7 +494,7 @@ template <> struct ItemOf<AMDC_Q6_K> { using type = ItemQ6; };
 // row's first one again, inside the same wave's lines, and ignores it): no
 // branch joins them, so that a wait for an earlier load does not become a
 // wait for these.
-template <int KIND>
+template <int KIND, bool LAST = true>
 __device__ __forceinline__ void load_item(Item &it, const uint8_t *wr, u32 ng, u32 g, bool ok) {
   g = ok ? g : 0u;
   it.h = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_header_off(g)));
@@ -502,22 +502,30 @@ __device__ __forceinline__ void load_item(Item &it, const uint8_t *wr, u32 ng, u
   for (u32 k = 0; k < 8u; k++) it.n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_nib_off(ng, g, k)));
 }
 
-template <int KIND>
+// Q8_0 / Q6_K: nontemporal (last) only where a row is whole 128-byte lines. In other rows two loads share lines (neighbouring
+// planes, or the ends of two rows), and a line taken nontemporally was gone before its second load. Measured on
+// MI355X (us, a Q8 vector, nontemporal / not; the persistent form): Q8_0 36000 x 11008 83.6 / 71.0 (74.0), 13000 x
+// 4608 16.8 / 15.4 (20.2), Q6_K 36000 x 13312 79.3 / 68 (72.1); whole lines: Q8_0 13000 x 4096 13.5 / 14.7 (16.1),
+// Q6_K 36000 x 7168 36.0 / 39.1 (41.2)
+template <bool LAST> __device__ __forceinline__ u32x4 load16(const uint8_t *p) {
+  return LAST ? __builtin_nontemporal_load((const u32x4 *)p) : *(const u32x4 *)p;
+}
+template <int KIND, bool LAST>
 __device__ __forceinline__ void load_item(ItemQ8 &it, const uint8_t *wr, u32 ng, u32 g, bool ok) {
   g = ok ? g : 0u;
-  it.h = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_header_off(g)));
+  it.h = load16<LAST>(wr + amdc_header_off(g));
 #pragma unroll
-  for (u32 k = 0; k < 16u; k++) it.n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_q8_off(ng, g, k)));
+  for (u32 k = 0; k < 16u; k++) it.n[k] = load16<LAST>(wr + amdc_q8_off(ng, g, k));
 }
-template <int KIND>
+template <int KIND, bool LAST>
 __device__ __forceinline__ void load_item(ItemQ6 &it, const uint8_t *wr, u32 ng, u32 g, bool ok) {
   g = ok ? g : 0u;
-  it.h = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_header_off(g)));
+  it.h = load16<LAST>(wr + amdc_header_off(g));
   it.d = *(const unsigned short *)(wr + amdc_q6k_d_off(ng, g));
 #pragma unroll
-  for (u32 k = 0; k < 8u; k++) it.n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_q6k_nib_off(ng, g, k)));
+  for (u32 k = 0; k < 8u; k++) it.n[k] = load16<LAST>(wr + amdc_q6k_nib_off(ng, g, k));
 #pragma unroll
-  for (u32 k = 0; k < 4u; k++) it.x[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_q6k_hi_off(ng, g, k)));
+  for (u32 k = 0; k < 4u; k++) it.x[k] = load16<LAST>(wr + amdc_q6k_hi_off(ng, g, k));
 }
 
 // One super-group's contribution to a row: for each of its 8 blocks k (LDS
@@ -799,7 +807,7 @@ __device__ __forceinline__ void norm_tail(const float *__restrict__ y, u32 rows,
   }
 }
 
-template <int KIND, u32 NI, bool FQ, u32 NTH, u32 QCN = 0u, bool TAIL = false>
+template <int KIND, u32 NI, bool FQ, u32 NTH, u32 QCN = 0u, bool TAIL = false, bool LAST = true>
 __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const uint8_t *__restrict__ xq, float *__restrict__ y, u32 rows,
                                            u32 nb, const float *__restrict__ bias, const float *__restrict__ res, u32 L,
                                            const float *__restrict__ xf = nullptr, uint8_t *__restrict__ q8out = nullptr,
@@ -870,7 +878,7 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
     for (u32 k = 0; k < PB; k++) it[0].n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_nib_off(ng, g, k)));
   } else {
 #pragma unroll
-    for (u32 i = 0; i < NI0; i++) load_item<KIND>(it[i], wr, ng, l + L * i, l + L * i < ng);
+    for (u32 i = 0; i < NI0; i++) load_item<KIND, LAST>(it[i], wr, ng, l + L * i, l + L * i < ng);
   }
   if (FQ) {
     fq.quant(0, nb, ng, s_lo, s_hi, s_d, s_as, q8out);
@@ -884,7 +892,7 @@ __device__ __forceinline__ void gemvs_body(const uint8_t *__restrict__ W, const 
       for (u32 k = PB; k < 8u; k++) it[0].n[k] = __builtin_nontemporal_load((const u32x4 *)(wr + amdc_nib_off(ng, g, k)));
     }
 #pragma unroll
-    for (u32 i = NI0; i < NI; i++) load_item<KIND>(it[i], wr, ng, l + L * i, l + L * i < ng);
+    for (u32 i = NI0; i < NI; i++) load_item<KIND, LAST>(it[i], wr, ng, l + L * i, l + L * i < ng);
   } else {
 #pragma unroll
     for (u32 c = 0; c < NSV; c++) {
@@ -1268,12 +1276,33 @@ extern "C" __global__ __launch_bounds__(256) void amdc_gemv_q6_k_p2(const uint8_
 // all out at once, 97 to 127 VGPRs hold 4 or 5 waves per SIMD where the form above holds two items and 2 waves.
 // Measured on MI355X (us, f32 vector: quantize launch and the form above / this): Q8_0 2048 x 2048 6.8 / 3.9, 11264 x
 // 2048 10.9 / 6.7, 32000 x 2048 16.5 / 12.7, 4096 x 4096 9.1 / 5.8; Q6_K 6144 x 2048 8.4 / 5.3, 1024 x 5120 6.9 / 5.6,
-// 4096 x 4096 8.8 / 5.9; with the quantize launch kept (long rows): Q8_0 4096 x 11008 14.8 / 13.4, 152064 x 5120 140 /
-// 127, Q6_K 4096 x 11008 14.5 / 12.1 (5120 x 17408 22.5 / 25.4, 152064 x 5120 110.7 / 117: not taken); on a Q8 vector
-// Q6_K 100000 x 2048 46.0 / 31.7, Q8_0 100000 x 2048 60.2 / 32.8, 36000 x 8192 51.6 / 45.7
-GEMVS_KERNELS(q8_0, AMDC_Q8_0, 1, s, 256)
-GEMVS_KERNELS(q6_k, AMDC_Q6_K, 1, s, 256)
-GEMVS_KERNELS(q8_0, AMDC_Q8_0, 2, s, 256)
+// 4096 x 4096 8.8 / 5.9; with the quantize launch kept (long rows): Q8_0 4096 x 11008 14.8 / 12.5, 9919 x 5184 17.3 / 14.2,
+// 152064 x 5120 140 / 134, Q6_K 4096 x 11008 14.5 / 12.1, 152064 x 5120 115 / 106; on a Q8 vector Q6_K 100000 x 2048 46.0 /
+// 31.7, Q8_0 100000 x 2048 60.2 / 32.8, 36000 x 8192 51.6 / 45.7
+#define GEMVS8_KERNEL(KN, KIND, NI, TAG, LAST)                                                                                        \
+  extern "C" __global__ __launch_bounds__(256) void amdc_gemv_##KN##_s##TAG(const uint8_t *W, const uint8_t *xq, float *y, u32 rows,  \
+                                                                            u32 nb, const float *bias, const float *res, u32 L) {    \
+    gemvs_body<KIND, NI, false, 256u, 0u, false, LAST>(W, xq, y, rows, nb, bias, res, L);                                              \
+  }
+#define GEMVXS8_KERNEL(KN, KIND, NI, TAG, LAST)                                                                                       \
+  extern "C" __global__ __launch_bounds__(256) void amdc_gemv_##KN##_xs##TAG(const uint8_t *W, const float *x, float *y, u32 rows,    \
+                                                                             u32 nb, const float *bias, const float *res, u32 L,     \
+                                                                             uint8_t *q8) {                                          \
+    gemvs_body<KIND, NI, true, 256u, 0u, false, LAST>(W, nullptr, y, rows, nb, bias, res, L, x, q8);                                   \
+  }
+// (_s1l, ...: nontemporal loads; two kernels and no branch between them, which took amdc_gemv_q6_k_xs1 from
+// 97 to 127 VGPRs)
+GEMVS8_KERNEL(q8_0, AMDC_Q8_0, 1, 1, false)
+GEMVS8_KERNEL(q8_0, AMDC_Q8_0, 1, 1l, true)
+GEMVXS8_KERNEL(q8_0, AMDC_Q8_0, 1, 1, false)
+GEMVXS8_KERNEL(q8_0, AMDC_Q8_0, 1, 1l, true)
+GEMVS8_KERNEL(q8_0, AMDC_Q8_0, 2, 2, false)
+GEMVS8_KERNEL(q8_0, AMDC_Q8_0, 2, 2l, true)
+GEMVXS8_KERNEL(q8_0, AMDC_Q8_0, 2, 2l, true) // (on half the lanes of a row of 16 or a multiple: whole lines)
+GEMVS8_KERNEL(q6_k, AMDC_Q6_K, 1, 1, false)
+GEMVS8_KERNEL(q6_k, AMDC_Q6_K, 1, 1l, true)
+GEMVXS8_KERNEL(q6_k, AMDC_Q6_K, 1, 1, false)
+GEMVXS8_KERNEL(q6_k, AMDC_Q6_K, 1, 1l, true)
 // the Q8_0 / Q6_K decode form with the fused RMSNorm tail (amdc_gemv_norm)
 #define GEMV2N_KERNEL(KN, KIND)                                                                                                      \
   extern "C" __global__ __launch_bounds__(256) void amdc_gemv_##KN##_pn(const uint8_t *W, const uint8_t *xq, float *y, u32 rows,    \
