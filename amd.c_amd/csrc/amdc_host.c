@@ -220,7 +220,6 @@ static struct {
   hipError_t (*StreamDestroy)(hipStream_t);
   hipError_t (*StreamSynchronize)(hipStream_t);
   hipError_t (*StreamWaitEvent)(hipStream_t, hipEvent_t, unsigned);
-  hipError_t (*StreamIsCapturing)(hipStream_t, int *);
   hipError_t (*StreamBeginCapture)(hipStream_t, int);
   hipError_t (*StreamEndCapture)(hipStream_t, hipGraph_t *);
   hipError_t (*GraphInstantiate)(hipGraphExec_t *, hipGraph_t, void *, char *, size_t);
@@ -405,7 +404,6 @@ static int hip_load(void) {
   SYM(StreamDestroy, "hipStreamDestroy");
   SYM(StreamSynchronize, "hipStreamSynchronize");
   SYM(StreamWaitEvent, "hipStreamWaitEvent");
-  SYM(StreamIsCapturing, "hipStreamIsCapturing");
   SYM(StreamBeginCapture, "hipStreamBeginCapture");
   SYM(StreamEndCapture, "hipStreamEndCapture");
   SYM(GraphInstantiate, "hipGraphInstantiate");
@@ -763,15 +761,11 @@ static u32 gemv2_lanes(u32 ng, u32 rows, int k8) {
 #define GEMV_LDS_T1 (150u * 1024u)
 
 static int ws_take(size_t n, void **p);
-/* Whether n bytes of workspace are there, or can be allocated: not while the stream is captured. The Q6_K
- * choices that need a workspace where others do not (a K split of at most 4 tiles, the verify kernel in place of
- * amdc_gemv_q6_k_m1) ask it, so that those calls can always be captured. */
-static int ws_ready(size_t n, void *stream);
 
 /* The verify GEMV on int8 MFMA (T <= 16): 64 rows per workgroup, K split
  * over aligned ranges of tiles (64 blocks each): for T <= 8 until the
  * workgroups fill the resident slots about once (Q4 kinds) or the CUs four
- * times (Q8_0), for T > 8 and Q6_K by an estimate of the time. A range holds S
+ * times (Q8_0, Q6_K), for T > 8 by an estimate of the time. A range holds S
  * tiles, S a power of two <= 4, so that its sum is a subtree of the
  * super-group tree (the kernels' order, equal to the decode GEMV's) and the
  * split sums' tree over the ranges (in the kernel for T <= 8, else
@@ -794,7 +788,7 @@ static int gemv8_launch(int kind, const void *w, const uint8_t *xq, float *y, ui
   if (want > 16u) want = 16u; /* amdc_gemm_reduce adds at most 16 ranges */
   u32 tps = 1;
   while (tps < 4u && tps * want < nt) tps <<= 1; /* the smallest S with ceil(nt / S) <= want (nt <= 32: S <= 2 for 16) */
-  if (T > 8u && t_ksplit <= 0 && wgs < 2u * cus && kind != AMDC_KIND_Q6_K) {
+  if (T > 8u && t_ksplit <= 0 && wgs < 2u * cus) {
     /* the 16-vector kernels hold one workgroup per CU: the range size S (1, 2, 4 tiles) with the fewest
        tile times, (rounds of workgroups) x S, plus one for the reduction launch of a split; ties to the
        larger S (grids of two workgroups per CU and more are not split). Measured on MI355X (T = 16, us): 11008 x 4096 Q4_0 16.7 unsplit against 20.8 in 2 splits,
@@ -815,21 +809,22 @@ static int gemv8_launch(int kind, const void *w, const uint8_t *xq, float *y, ui
   /* T <= 8, 2 tiles of K and at least half a workgroup per CU: unsplit (MI355X, T = 8, us: 11008 x
      4096 Q8_0 14.3 against 15.2-15.4 in 2 splits, Q4_0 12.2 against 12.3) */
   if (T <= 8u && nt == 2u && t_ksplit <= 0 && 2u * wgs >= cus) tps = 2u;
-  if (kind == AMDC_KIND_Q6_K && t_ksplit <= 0) {
-    /* Q6_K, any T: two workgroups per CU; the range size S with the fewest tile times, rounds (at least one, else
-       as many as the workgroups are of the resident ones) x S, plus one for a split's sums; ties to the smaller S.
-       Measured on MI355X (us, S = 1, 2, 4, T = 16): 5120 x 17408 35.7 / 36.7 / 50.9, 17408 x 5120 37.4 / 37.7 / 46.6,
-       20480 x 8192 52 / 57 / 62, 32000 x 4096 42 / 34 unsplit, 11008 x 4096 22 / 26.7 unsplit; T = 8 alike */
+  /* Q6_K: two workgroups per CU also for T > 8, so where the rules above split, the range size S with the fewest tile
+     times: T <= 8 a workgroup's S tiles and one to start, or all of them on the resident ones if that is more; T > 8
+     rounds (at least one) x S; half or one for a split's sums; ties to the smaller S. Calls that run unsplit by the rules
+     above stay so: they use no workspace, and may overlap on the device (MI355X, us, unsplit / split, T = 16 4096 x 4096
+     25.7 / 17.2, T = 8 11008 x 4096 18.5 / 17.8). Measured (us, S = 1, 2, 4): T = 4 16000 x 17408 69.1 / 62.4 / 58.5, 8192 x 17408
+     39.1 / 36.0 / 46.0, 5120 x 17408 26.1 / 26.4 / 33.4; T = 16 5120 x 17408 35.7 / 36.7 / 50.9, 17408 x 5120 37.4 / 37.7 / 46.6 */
+  if (kind == AMDC_KIND_Q6_K && t_ksplit <= 0 && tps < nt && wgs < 2u * cus) {
     const double slots = 2.0 * cus;
     double best = 1e30;
-    tps = 4u;
-    for (u32 S = 4u; S >= 1u && wgs < 2u * cus; S >>= 1) {
-      const u32 n = (nt + S - 1u) / S;
+    for (u32 S = 4u; S >= 1u; S >>= 1) {
+      const u32 n = (nt + S - 1u) / S, s = S < nt ? S : nt;
       if (n > 16u) break;
-      const double r = (double)wgs * n / slots, est = (r > 1.0 ? r : 1.0) * (S < nt ? S : nt) + (n > 1u ? 1.0 : 0.0);
+      const double all = (double)wgs * (nt + n) / slots, r = (double)wgs * n / slots;
+      const double est = (T <= 8u ? (all > s + 1u ? all : s + 1u) : (r > 1.0 ? r : 1.0) * s) + (n > 1u ? (T <= 8u ? 0.5 : 1.0) : 0.0);
       if (est <= best) best = est, tps = S;
     }
-    if (nt <= 4u && !ws_ready((size_t)((nt + tps - 1u) / tps) * T * rows * 4u, stream)) tps = 4u;
   }
   const u32 ks = (nt + tps - 1u) / tps;
   float *part = NULL;
@@ -1000,11 +995,11 @@ static int gemv_launch(int kind, const void *w, const uint8_t *xq, float *y, uin
       /* measured on MI355X (us, this kernel / the MFMA verify kernel): Q6_K 1024 x 5120 T = 2, 4, 8 5.5 /
          10.9, 7.1 / 10.8, 10.5 / 11.3; 4096 x 4096 6.8 / 12.1, 8.5 / 12.2, 11.7 / 12.7; 6144 x 5120 T = 4, 6
          15.5 / 15.8, 18.7 / 16.2; 11008 x 4096 T = 4 16.8 / 17.1; 4096 x 11008 (43 of 64 lanes) T = 4 21.0 /
-         17.6; 17408 x 5120 T = 2 25.1 / 28.7: Q6_K past T = 2 counts its idle lanes too. Q8_0 4096 x 4096 6.4 / 9.5, 7.8 / 9.6, 10.6 / 10.1; 11008 x 4096 T = 2, 4 12.3 /
+         17.6; 17408 x 5120 T = 2 25.1 / 28.7: Q6_K also a little past where the other is as fast (a call here uses no
+         workspace, and may overlap others on the device). Q8_0 4096 x 4096 6.4 / 9.5, 7.8 / 9.6, 10.6 / 10.1; 11008 x 4096 T = 2, 4 12.3 /
          15.2, 15.4 / 14.9; 1024 x 2048 T = 8 7.6 / 6.5: Q8_0 only up to T = 4 and half the size */
       const u64 lim = kind == AMDC_KIND_Q6_K ? M8_MAX : T <= 4u ? M8_MAX * 2u / 3u : 0u;
-      const u32 gl = kind == AMDC_KIND_Q6_K && T > 2u && ws_ready((size_t)16u * T * rows * 4u, stream) ? L : ng;
-      if (ni == 1u && lds <= 64u * 1024u && (u64)T * rows * gl <= lim && (u64)rows * rb + rb < (1ull << 32)) {
+      if (ni == 1u && lds <= 64u * 1024u && (u64)T * rows * ng <= lim && (u64)rows * rb + rb < (1ull << 32)) {
         void *a[] = {&w, &xq, &y, &rows, &nb, &bias, &res, (void *)&L, &T, &xs, &ys, &rs};
         return launch(K_GEMVM8 + (kind == AMDC_KIND_Q6_K ? 1 : 0), nrg, 1, lds, stream, a);
       }
@@ -1306,12 +1301,6 @@ static int ws_reserve(size_t n) {
   HIPCALL(H.Malloc(&g_ws, m));
   g_ws_bytes = m;
   return AMDC_OK;
-}
-
-static int ws_ready(size_t n, void *stream) {
-  int st = 0; /* hipStreamCaptureStatusNone */
-  if (n <= (g_ws_fixed ? g_scratch_bytes : g_ws_bytes)) return 1;
-  return !g_ws_fixed && (!stream || (H.StreamIsCapturing(stream, &st) == 0 && st == 0));
 }
 
 /* The workspace of an operator: n bytes at *p, from the grown allocation, or from the fixed
