@@ -1446,20 +1446,22 @@ static int gemm_launch(int kind, const char *op, const void *w, const uint8_t *x
     void *args[] = {&w, &xq, &y, &rows, &nb, &bias, &res, &T, &xs, &ys, &rs};
     return launch(n == 128u ? K_GEMM_N128 : K_GEMM_N64, (unsigned)grid, 1, 0, stream, args);
   }
-  /* the wide-tile kernels, above 2^22 weights times token tiles of 64: below that the 64-row kernels' shorter way to the
-     first product wins (MI355X, us, 64-row / wide: 1000 x 4096 Q4_K T = 33 13.6 / 16.9, 2048 x 2048 Q6_K T = 64
-     16.1 / 19.5, 4096 x 1024 Q8_0 T = 20 12.8 / 14.9; above, 2048 x 4096 Q4_0 T = 33 18.4 / 16.2, 1000 x 8192 Q4_K T = 64
-     19.7 / 19.8, 4096 x 4096 Q4_K T = 33 27.3 / 19.0) */
-  const int small = (u64)rows * nb * 32u * ((T + 63u) / 64u) <= (1ull << 22);
+  /* the wide-tile kernels, above 2^22 weights times token tiles of 64 (Q4_K up to 64 tokens: 6.3 million weights; 65 to 96
+     tokens, a tile and a half, on matrices of 2^21 to 2^22 weights: the 64-row kernel's 128-token tile). Below that the 64-row
+     kernels' shorter way to the first product wins (MI355X, us, 64-row / wide: 1000 x 4096 Q4_K T = 33 13.6 / 16.9, 2048 x
+     2048 Q6_K T = 64 16.1 / 19.5, 4096 x 1024 Q8_0 T = 20 12.8 / 14.9, 4096 x 1536 Q4_K T = 33 15.7 / 17.1, 2048 x 3072 T = 20
+     14.7 / 16.5; T = 65 1400 x 2048 Q8_0 18.0 / 20.0, Q6_K 18.2 / 20.5, Q4_K 16.4 / 18.8; above, 2048 x 4096 Q4_0 T = 33 18.4 / 16.2,
+     1000 x 8192 Q4_K T = 64 19.7 / 19.8, 4096 x 4096 Q4_K T = 33 27.3 / 19.0, 1400 x 3072 Q8_0 T = 65 23.0 / 21.0) */
+  const u64 nw = (u64)rows * nb * 32u;
+  const int mid = T > 64u && T <= 96u && kind != AMDC_KIND_Q4_0 && nw > (1u << 21) && nw <= (1u << 22);
+  const int small = mid || nw * ((T + 63u) / 64u) <= (kind == AMDC_KIND_Q4_K && T <= 64u ? 3u << 21 : 1u << 22);
   if (t_gemm == 5 || (t_gemm == 0 && !small)) {
     if ((rc = gemmw_launch(kind, w, xq, y, rows, nb, bias, res, T, xs, ys, rs, stream)) != -1) return rc;
     rc = AMDC_OK;
   }
-  /* the 64-row f16-MFMA kernels: 128 tokens per workgroup when there are that many; 64-token tiles for Q4_0 at any
-     T (its 128-token kernel holds 284 VGPRs, one wave per SIMD: measured 150 / 188 TOPS against 140 / 169 on 11008 x
-     4096 / 4096 x 11008, T = 256) */
+  /* the 64-row f16-MFMA kernels: 64-token tiles (small matrices: T = 128 1000 x 2048 Q8_0 64 / 128 tokens 16.9 / 19.5 us), but for mid */
   const u32 ng = amdc_ngroups(nb), cus = g_cus > 0 ? (u32)g_cus : 256u;
-  const int v = t_gemm == 3 || t_gemm == 4 ? t_gemm - 3 : (T > 64u && kind != AMDC_KIND_Q4_0 && !small ? 0 : 1);
+  const int v = t_gemm == 3 || t_gemm == 4 ? t_gemm - 3 : mid ? 0 : 1;
   const int kk = kind == AMDC_KIND_Q8_0 ? (v ? K_GEMMH_Q8_N64 : K_GEMMH_Q8_N128)
                  : kind == AMDC_KIND_Q6_K ? (v ? K_GEMMH_Q6K_N64 : K_GEMMH_Q6K_N128)
                  : kind == AMDC_KIND_Q4_0 ? (v ? K_GEMMH_Q4_N64 : K_GEMMH_Q4_N128)
