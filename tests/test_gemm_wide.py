@@ -17,16 +17,18 @@ KINDS = [synth.KIND_Q4_0, synth.KIND_Q8_0, synth.KIND_Q4_K, synth.KIND_Q6_K]
 # last), tokens around 64 and 128, splits that leave a workgroup a single super-group
 @pytest.mark.parametrize("rows,nb,T,ks", [(1, 8, 33, 0), (127, 16, 63, 0), (128, 24, 64, 0), (129, 40, 65, 0), (257, 24, 128, 2),
                                           (300, 72, 129, 3), (130, 104, 200, 7)])
-def test_edges(dev, orc, kind, rows, nb, T, ks):
+@pytest.mark.parametrize("kern", [0, 5])  # as dispatched (the 64-row kernels at these sizes), and the wide tiles
+def test_edges(dev, orc, kind, rows, nb, T, ks, kern):
     c = Case(dev, orc, kind, rows, nb, T, seed=rows + T)
     c.quant()
     g = np.random.default_rng(T)
     bias, res = g.standard_normal(rows).astype(np.float32), g.standard_normal((T, rows)).astype(np.float32)
     B, R = dev.DevBuf.of(bias), dev.DevBuf.of(res)
-    dev.set_tuning(gemm_ksplit=ks)
+    dev.set_tuning(gemm_kernel=kern, gemm_ksplit=ks)
     try:
         c.Y.fill(0xFF)
         dev.gemm(kind, c.W, c.Q, c.Y, rows, nb, T, c.xs, rows, rows, bias=B, res=R)
+        assert dev.last_kernel() == "amdc_gemm_reduce" or dev.last_kernel().startswith("amdc_gemmw" if kern else "amdc_gemmh")
     finally:
         dev.set_tuning()
     y = c.y_gpu()
@@ -38,12 +40,18 @@ def test_edges(dev, orc, kind, rows, nb, T, ks):
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", [synth.KIND_Q4_0, synth.KIND_Q8_0])
 @pytest.mark.parametrize("nb", [1, 7, 9, 21])
-def test_ragged_blocks(dev, orc, kind, nb):
+@pytest.mark.parametrize("T,kern", [(70, 0), (40, 5), (70, 5)])
+def test_ragged_blocks(dev, orc, kind, nb, T, kern):
     """Rows whose last super-group is partly filled."""
-    rows, T = 140, 70
+    rows = 140
     c = Case(dev, orc, kind, rows, nb, T, seed=nb)
     c.quant()
-    dev.gemm(kind, c.W, c.Q, c.Y, rows, nb, T, c.xs, rows)
+    c.Y.fill(0xFF)
+    dev.set_tuning(gemm_kernel=kern)
+    try:
+        dev.gemm(kind, c.W, c.Q, c.Y, rows, nb, T, c.xs, rows)
+    finally:
+        dev.set_tuning()
     y = c.y_gpu()
     for t in range(T):
         assert rel_err(y[t], c.y_oracle(t), c.mag(t)) < TOL, t
@@ -52,8 +60,8 @@ def test_ragged_blocks(dev, orc, kind, nb):
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", KINDS)
 def test_many_tiles_exact(dev, orc, kind):
-    """More tiles than the device holds at once (the third form for all but Q8_0: whole rounds and a split tail)
-    against the exact sums, spot-checked over every row and token tile."""
+    """More tiles than the device holds at once (128 tokens in two groups, unsplit) against the exact sums, spot-checked over
+    every row and token tile."""
     rows, nb, T = 128 * 130 + 5, 16, 128 * 4 + 3
     src = exactcase.gguf(kind, rows, 32 * nb, seed=kind)
     x = exactcase.activations(T, 32 * nb, seed=kind + 1)
@@ -67,6 +75,64 @@ def test_many_tiles_exact(dev, orc, kind):
     for t in range(0, T, 37):
         assert np.array_equal(y[t], exactcase.exact_y(orc, kind, src, rows, nb, xq[t])), t
     assert np.isfinite(y).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [synth.KIND_Q4_0, synth.KIND_Q4_K, synth.KIND_Q6_K])
+@pytest.mark.parametrize("nb", [16, 24])
+def test_two_workgroups_exact(dev, orc, kind, nb):
+    """Two workgroups per CU (amdc_gemmw_*_i128; test_host_choice.py: these sizes take it): whole rounds of 170 row tiles x 3
+    token tiles and two row tiles in as many splits as super-groups, the last row tile and token tile ragged; against the
+    exact sums, and rows in strides with a bias and a residual."""
+    rows, T, ys, rs = 22003, 257, 22016, 22010
+    src = exactcase.gguf(kind, rows, 32 * nb, seed=kind + nb)
+    x = exactcase.activations(T, 32 * nb, seed=nb)
+    xs = (40 * nb + 255) // 256 * 256
+    g = np.random.default_rng(nb)
+    bias, res = g.integers(-9, 10, rows).astype(np.float32), g.integers(-9, 10, (T, rs)).astype(np.float32)
+    W, X, Q, Y, B, R = (dev.DevBuf.of(dev.repack(kind, src, rows, 32 * nb)), dev.DevBuf.of(x), dev.DevBuf(T * xs), dev.DevBuf(4 * T * ys),
+                        dev.DevBuf.of(bias), dev.DevBuf.of(res))
+    dev.quant_q8(X, Q, nb, T, 128 * nb, xs)
+    xq = orc.quant_q8(x)
+    Y.fill(0xFF)
+    dev.gemm(kind, W, Q, Y, rows, nb, T, xs, rows)
+    y = Y.download(np.float32)[:T * rows].reshape(T, rows).copy()
+    assert np.isfinite(y).all()
+    Y.fill(0xEE)
+    dev.gemm(kind, W, Q, Y, rows, nb, T, xs, ys, rs, bias=B, res=R)
+    z = Y.download(np.float32).reshape(T, ys)
+    assert (z[:, rows:].view(np.uint32) == 0xEEEEEEEE).all()
+    assert np.array_equal(z[:, :rows], res[:, :rows] + (y + bias))
+    for t in (0, 1, 63, 64, 127, 128, 191, 255, 256):
+        assert np.array_equal(y[t], exactcase.exact_y(orc, kind, src, rows, nb, xq[t])), t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("kern", [4, 5])
+@pytest.mark.parametrize("T", [40, 70, 150])
+@pytest.mark.parametrize("ks", [1, 2])  # whole K, every tile split
+def test_strides(dev, orc, kind, kern, T, ks):
+    """Rows of y, res and xq further apart than they are long: the bits of the packed call, nothing written between."""
+    rows, nb, ys, rs = 140, 24, 160, 150
+    c = Case(dev, orc, kind, rows, nb, T, seed=T)
+    c.quant()
+    g = np.random.default_rng(T)
+    bias, res = g.standard_normal(rows).astype(np.float32), g.standard_normal((T, rs)).astype(np.float32)
+    xs = c.xs + 272
+    q = np.full((T, xs), 0x5A, np.uint8)
+    q[:, :40 * nb] = c.xq
+    B, R, RP, Q, Y = dev.DevBuf.of(bias), dev.DevBuf.of(res), dev.DevBuf.of(np.ascontiguousarray(res[:, :rows])), dev.DevBuf.of(q), dev.DevBuf(4 * T * ys)
+    dev.set_tuning(gemm_kernel=kern, gemm_ksplit=ks)
+    try:
+        dev.gemm(kind, c.W, c.Q, c.Y, rows, nb, T, c.xs, rows, rows, bias=B, res=RP)
+        Y.fill(0xEE)
+        dev.gemm(kind, c.W, Q, Y, rows, nb, T, xs, ys, rs, bias=B, res=R)
+    finally:
+        dev.set_tuning()
+    z = Y.download(np.uint32).reshape(T, ys)
+    assert (z[:, rows:] == 0xEEEEEEEE).all()
+    assert np.array_equal(z[:, :rows], c.Y.download(np.uint32).reshape(T, rows))
 
 
 @pytest.mark.gpu

@@ -131,7 +131,8 @@ def test_errors_do_not_launch(dev, orc):
                                             (Q6, 1, 8, 17), (Q6, 63, 16, 64), (Q6, 64, 160, 65), (Q6, 130, 40, 130), (Q6, 70, 544, 33),
                                             (0, 1, 1, 17), (0, 63, 13, 64), (0, 130, 128, 65), (0, 70, 344, 33), (0, 300, 40, 256)])
 @pytest.mark.parametrize("ks", [0, 3])
-def test_gemm(dev, orc, kind, rows, nb, T, ks):
+@pytest.mark.parametrize("kern", [0, 5])  # as dispatched, and the wide tiles at these sizes
+def test_gemm(dev, orc, kind, rows, nb, T, ks, kern):
     """The prefill GEMM (f16 MFMA, exact integer block sums) against the oracle per token row, with a
     bias, with and without split K; Q8_0, Q6_K and the Q4_0 form (no reference kernel: the reference
     runs one GEMV per token)."""
@@ -142,7 +143,7 @@ def test_gemm(dev, orc, kind, rows, nb, T, ks):
         pytest.skip("fewer super-groups than splits")
     bias = np.random.default_rng(T).standard_normal(rows).astype(np.float32)
     B = dev.DevBuf.of(bias)
-    dev.set_tuning(gemm_ksplit=ks)
+    dev.set_tuning(gemm_kernel=kern, gemm_ksplit=ks)
     dev.gemm(kind, c.W, c.Q, c.Y, rows, nb, T, c.xs, rows, bias=B)
     y = c.y_gpu()
     for t in range(T):
@@ -150,7 +151,8 @@ def test_gemm(dev, orc, kind, rows, nb, T, ks):
 
 
 @pytest.mark.parametrize("kind", [Q8, Q6])
-def test_gemm_extreme_values(dev, orc, kind):
+@pytest.mark.parametrize("kern", [0, 5])
+def test_gemm_extreme_values(dev, orc, kind, kern):
     """Weights and activations at the ends of their ranges, where the exactness of the f16 sums is
     tightest: Q6_K q = 0 (q - 32 = -32) with scales -128 / 127, Q8_0 weights -128 / 127; activations
     of one block all +-127 (x = +-1)."""
@@ -177,6 +179,7 @@ def test_gemm_extreme_values(dev, orc, kind):
     c.Q = dev.DevBuf(T * c.xs)
     c.Y = dev.DevBuf(T * rows * 4)
     assert np.array_equal(c.quant(), c.xq)
+    dev.set_tuning(gemm_kernel=kern)
     dev.gemm(kind, c.W, c.Q, c.Y, rows, nb, T, c.xs, rows)
     y = c.y_gpu()
     for t in range(T):

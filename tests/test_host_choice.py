@@ -70,3 +70,10 @@ def test_gemm_kernel(stub):
             ((Q8, 1400, 64, 97), "gemmw_q8_0_"), ((Q6, 1024, 64, 128), "gemmh_q6_k_m64_n64"), ((Q4K, 1025, 64, 128), "gemmw_q4_k_")]
     for (call, kernel), (_, names) in zip(want, launched(stub, [("gemm",) + c for c, _ in want])):
         assert any(n.startswith(kernel) for n in names), (call, kernel, names)
+
+
+def test_two_workgroups(stub):
+    """22003 rows, 257 tokens: two workgroups per CU, whole rounds and a split tail (test_gemm_wide.py runs them)."""
+    kinds = {Q4: "q4_0", Q4K: "q4_k", Q6: "q6_k"}
+    calls = [("gemm", k, 22003, nb, 257) for k in kinds for nb in (16, 24)]
+    assert [n for _, n in launched(stub, calls)] == [["gemmw_prep", f"gemmw_{kinds[c[1]]}_i128", "gemm_reduce"] for c in calls]

@@ -11,21 +11,23 @@ what the kernels rely on but the compiler cannot see:
 * the integer block dots run on v_dot4_i32_i8 in the decode kernels, and the
   verify and prefill kernels run on MFMA;
 * every buffer load into the LDS has at least one instruction between the
-  write of m0 that addresses it and the load (the gfx9 hazard); in the verify
-  kernels whose LDS loads are inline asm (lds_load16), m0 is written only right
-  before such a load;
-* the explicit waits of those kernels and of the Q6_K verify kernels (vm_wait,
-  marked by expcnt(6)): a plane's
+  write of m0 that addresses it and the load (the gfx9 hazard); in the kernels
+  whose LDS loads are inline asm (lds_load16: the verify kernels and the wide-tile
+  GEMM), m0 is written only right before such a load;
+* the explicit waits of those kernels (vm_wait, marked by expcnt(6)). Verify: a plane's
   ring slot was filled by a load into the LDS issued one ring step earlier,
   and the count n of the wait must leave that load complete, i.e. at least n
   vector memory instructions were issued after it. The check walks the
   compiled instruction order, on the first pass through the tile loop (after
-  the prologue) and in the steady state (after the previous iteration).
+  the prologue) and in the steady state (after the previous iteration). Wide-tile
+  GEMM: a stage's wait leaves at most as many loads in flight as the stage after it
+  has issued at least (loads that only some waves issue are not counted).
 """
 import os
 import re
 import shutil
 import subprocess
+from collections import deque
 
 import pytest
 
@@ -43,13 +45,14 @@ INLINE_LDS = {
     "amdc_gemv_q4_0_v16": (2, 1, 8),
     "amdc_gemv_q4_k_v16": (2, 1, 8),
     "amdc_gemv_q8_0_v16": (1, 4, 8),
-}
-# kernels whose loads into the LDS are the compiler's builtin but whose ring reads wait explicitly:
-# gemv8_q6k_body<NQ, NS>: NS steps of 6 loads, a wait per step (4 per tile)
-BUILTIN_LDS = {
+    # gemv8_q6k_body<NH, NS>: NS steps of 6 loads, a wait per step (4 per tile)
     "amdc_gemv_q6_k_v8": (2, 6, 4),
     "amdc_gemv_q6_k_v16": (1, 6, 4),
 }
+# gemmw_body<KIND, NJ, GR>: the loads that a stage's wait may leave in flight (64-token tiles: a stage ahead, of which
+# every wave issues at least NF + NA / 4 loads; 128-token tiles: none)
+WIDE = {f"amdc_gemmw_{k}_{f}": (0 if f != "n64" else 4 if k == "q8_0" else 3)
+        for k in ("q4_0", "q4_k", "q6_k", "q8_0") for f in ("n128", "n64", "i128") if (k, f) != ("q8_0", "i128")}
 
 
 def _tool(name):
@@ -130,8 +133,8 @@ def test_decode_dots_on_dot4(code):
 
 def test_verify_and_gemm_on_mfma(code):
     funcs, _ = code
-    mm = [k for k in funcs if re.match(r"amdc_(gemv_\w+_v(8|16)|gemmh_\w+|gemm_q\w+)$", k)]
-    assert len(mm) >= 16
+    mm = [k for k in funcs if re.match(r"amdc_(gemv_\w+_v(8|16)|gemmh_\w+|gemmw_q\w+|gemm_q\w+)$", k)]
+    assert len(mm) >= 27 and set(WIDE) <= set(mm)
     for k in mm:
         assert any(mn.startswith("v_mfma_") for _, mn, _ in funcs[k]), k
 
@@ -151,7 +154,7 @@ def test_m0_hazard(code):
 def test_inline_lds_m0_only_for_the_load(code):
     """In the lds_load16 kernels m0 is set only as `s_mov_b32 m0; s_nop 0; buffer_load ... lds`."""
     funcs, _ = code
-    for k in INLINE_LDS:
+    for k in [*INLINE_LDS, *WIDE]:
         ins = funcs[k]
         loads = 0
         for i, (_, mn, ops) in enumerate(ins):
@@ -180,7 +183,7 @@ def _check_waits(name, seq, marks, ns, dps):
 
 def test_explicit_waits_cover_the_ring(code):
     funcs, _ = code
-    for k, (ns, dps, nw) in {**INLINE_LDS, **BUILTIN_LDS}.items():
+    for k, (ns, dps, nw) in INLINE_LDS.items():
         ins = funcs[k]
         marked = [i for i, (_, mn, ops) in enumerate(ins) if mn == "s_waitcnt" and "expcnt(6)" in ops]
         assert len(marked) == nw, f"{k}: {len(marked)} marked waits ({nw} per tile expected)"
@@ -195,6 +198,42 @@ def test_explicit_waits_cover_the_ring(code):
         # steady state: the body after the body
         two = body + body
         _check_waits(k, two, [len(body) + (i - s) for i in marked], ns, dps)
+
+
+def test_wide_gemm_waits(code):
+    funcs, _ = code
+    for k, left in WIDE.items():
+        ins = funcs[k]
+        marked = [i for i, (_, mn, ops) in enumerate(ins) if mn == "s_waitcnt" and "expcnt(6)" in ops]
+        count = [int(re.search(r"vmcnt\((\d+)\)", ins[i][2]).group(1)) for i in marked]
+        # the first stages, the four stages of the loop, and before the output
+        assert count == [0, left, left, left, left, 0], (k, count)
+        for n in range(1, 5):  # the loads issued after the wait of stage n, before that of the next
+            got = _fewest_lds(ins, marked[n], marked[n + 1] if n < 4 else marked[1], set(marked))
+            assert got >= left, f"{k}: after the wait at {ins[marked[n]][0]:#x} a wave may issue only {got} loads, the next wait leaves {left}"
+
+
+def _fewest_lds(ins, a, b, stops):
+    """The fewest loads into the LDS on any way through the code from instruction a to b that meets no other of stops."""
+    best, todo = {}, deque([(a, 0)])
+    while todo:
+        i, n = todo.popleft()
+        if i in best and best[i] <= n:
+            continue
+        best[i] = n
+        if i == b and i != a:
+            return n
+        if i in stops and i != a:
+            continue
+        mn = ins[i][1]
+        n += is_lds_dma(*ins[i][1:])
+        to = [_target(ins, i)] if mn.startswith(("s_branch", "s_cbranch")) else []
+        if not mn.startswith(("s_branch", "s_endpgm")):
+            to.append(i + 1)
+        for t in to:
+            if t is not None and t < len(ins):
+                (todo.append if n > best[i] else todo.appendleft)((t, n))
+    raise AssertionError("no way from one wait to the next")
 
 
 def _target(ins, i):
