@@ -1328,9 +1328,9 @@ static const struct {
 /* The prefill GEMM on the wide-tile kernels (amdc_gemmw_*): tiles of 128 rows x 128 or 64 tokens, in three
  * forms: a tile per CU (512 threads, the two halves of the workgroup taking the super-groups in turn) of 128 or
  * 64 tokens, and two independent 256-thread workgroups of 128 tokens per CU. Their measured cost per form, in
- * 0.1 us (MI355X, 34816 x 5120, T = 1000, the time of a round of resident workgroups less GW_ROUND): of two
- * super-groups for the first two forms, of one for the third, by gw_kind. Q8_0 does not take the third form:
- * its weight planes at 16 bytes a row outweigh it (512 tokens 360 us against 348). */
+ * 0.1 us (MI355X, 34816 x 5120, T = 1000, the time of a round of resident workgroups less GW_ROUND; the 64-token tiles
+ * in waves of 64 rows x 32 tokens, 3 to 10 % slower than now): of two super-groups for the first two forms, of one for
+ * the third, by gw_kind. Q8_0 does not take the third form: its weight planes at 16 bytes a row outweigh it (512 tokens 360 us against 348). */
 enum { GW_J128, GW_J64, GW_I128, GW_FORMS };
 #define GW_ROUND 40u  /* a round of workgroups: first loads, the tile's output */
 #define GW_REDUCE 40u /* the launch of the split sums */
@@ -1540,12 +1540,13 @@ int amdc_gemm_q6k(const void *w, const uint8_t *xq, float *y, uint32_t rows, uin
 }
 
 /* op_gemv's choice for T > 1: the prefill GEMM or the verify kernels (up to 16 vectors per
- * launch). IE_GEMM_MIN set (> 0): the reference's rule, T >= IE_GEMM_MIN. Else measured on
- * MI355X (us per call, verify / GEMM): the verify kernels win up to T = 32 on the 7B-27B layer
- * shapes (17408 x 5120 Q4_K T = 32: 60 / 70, T = 33: 70 / 70, T = 40: 79 / 71; 4096 x 11008
- * Q4_0 T = 32: 36 / 43; 5120 x 6144 Q4_K T = 32: 32 / 37), except on matrices of at most 2^24
- * weights, where the GEMM wins from T = 20 (4096 x 4096 Q4_0 T = 20: 27 / 23, T = 17: 19 / 22;
- * Q8_0 T = 20: 29 / 27). */
+ * launch). IE_GEMM_MIN set (> 0): the reference's rule, T >= IE_GEMM_MIN. Else from T = 33, and on matrices of at most 2^24
+ * weights from T = 20: the line of the GEMM and Q6_K verify kernels before the present ones. With these (MI355X, us
+ * per call, verify / GEMM) it holds for Q8_0 and Q6_K on large matrices and comes late for the Q4 kinds: T = 17, 24, 32
+ * 17408 x 5120 Q4_K 44 / 51, 51 / 52, 65 / 52; 32768 x 5120 Q4_0 65 / 57, 70 / 58, 92 / 59; 5120 x 17408 Q4_K 40 / 44,
+ * 43 / 44, 53 / 45; 4096 x 11008 Q4_0 25 / 25, 26 / 25, 30 / 26; 17408 x 5120 Q8_0 67 / 73, 74 / 73, 93 / 75; 5120 x 17408
+ * Q8_0 61 / 74, 64 / 74, 78 / 75; 17408 x 5120 Q6_K 52 / 69, 65 / 69, 72 / 71; 4096 x 4096 (16.8 million weights) T = 17, 20
+ * Q4_0 19 / 17, 22 / 17, Q8_0 27 / 19, 26 / 20, Q6_K 21 / 20, 24 / 20. */
 static int use_gemm(uint32_t T, uint32_t rows, uint32_t nb) {
   if (t_gemm_min > 0) return (int)T >= t_gemm_min;
   if (T >= 33u) return 1;

@@ -412,7 +412,8 @@ extern "C" __global__ __launch_bounds__(256) void amdc_swiglu_q8(float *__restri
 }
 
 // The same on 16-byte aligned rows of a and b and 4-byte aligned rows of q: 4 values per lane. Grid (ceil(n / 1024),
-// T). Measured on MI355X (us): n = 17408, T = 256 14.6 / 8.6, T = 8 2.4 / 2.3 (the form above / this)
+// T). Measured on MI355X (us): n = 17408, T = 256 14.8 / 8.3, T = 96 6.3 / 4.6, T = 32 3.6 / 3.0, T = 8 2.5 /
+// 2.4; n = 5120, T = 96 3.3 / 2.9, T = 16 2.4 / 2.4 (the form above / this)
 extern "C" __global__ __launch_bounds__(256) void amdc_swiglu_q8_v(float *__restrict__ a, const float *__restrict__ b, u32 n, uint8_t *__restrict__ q,
                                                                   u32 as, u32 qs) {
   a = (float *)((uint8_t *)a + (u64)blockIdx.y * as);
@@ -431,7 +432,7 @@ extern "C" __global__ __launch_bounds__(256) void amdc_swiglu_q8_v(float *__rest
 // amdc_rmsnorm_q8 with a workgroup per row, for many rows: the other form's n / 256 workgroups per row each read it
 // all for the sum of squares (the same code here, so the same s); then 4 values per lane, the row again from L1 / L2.
 // 16-byte aligned rows of x, y and w, 4-byte aligned rows of q. Grid (1, T). Measured on MI355X (us): n = 5120, T = 256 13.6 / 6.2,
-// T = 512 22.6 / 7.4, T = 64 4.4 / 5.4; n = 5376, T = 98 6.6 / 6.2; n = 4096, T = 128 4.8 / 4.6; n = 1024, T = 512
+// T = 512 22.6 / 7.4, T = 64 4.4 / 5.4; n = 5376, T = 98 6.6 / 6.2; n = 5120, 96 and 100 rows 5.3 / 5.3; n = 8192, T = 96 7.5 / 6.2; n = 4096, T = 128 4.8 / 4.6; n = 1024, T = 512
 // 4.7 / 3.6; 256, 2048 4.0 / 4.7; 8192, 64 6.0 / 7.0; 17408, 32 10.1 / 12.6 (the other form / this)
 extern "C" __global__ __launch_bounds__(256) void amdc_rmsnorm_q8_r(const float *__restrict__ x, const float *__restrict__ w, float *__restrict__ y,
                                                                    u32 n, float eps, uint8_t *__restrict__ q, u32 xs, u32 ys, u32 qs) {
@@ -3205,11 +3206,11 @@ __device__ __forceinline__ void a_frag_w6(u32 q0, u32 q1, h2 s, h8 &hi, h8 &lo) 
 // stage apart, and add their sums through the LDS at the end: both waves of a SIMD work on one tile where there are
 // only about as many tiles as CUs. GR = 1: a 256-thread workgroup per tile, two independent ones per CU, whose waits
 // overlap better (34816 x 5120 Q4_K, T = 1024: 617 against 675 us), for matrices of many tiles.
-// Measured on MI355X (us, whole call with the quantization, gemmh / this): 17408 x 5120 Q4_K T = 256 146.8 / 100.1,
-// 34816 x 5120 Q4_K T = 1024 1024 / 628 (582 TOPS), 11008 x 4096 Q4_0 T = 77 93.7 / 43.9, 5120 x 17408 Q6_K T = 256 236 /
-// 150, 4096 x 11008 Q8_0 T = 384 231 / 134. Its error against 64 bits is below gemmh's on each (1.4e-7 against 2.4e-7
-// for the first). With its loads from memory left out it took 463 of 617 us, with its LDS reads left out too 414; at
-// full load the card runs it at 2.0 GHz.
+// Measured on MI355X (us, whole call with the quantization, gemmh / this): 17408 x 5120 Q4_K T = 256 146.5 / 100.8,
+// 34816 x 5120 Q4_K T = 1024 1024 / 614 (595 TOPS), 11008 x 4096 Q4_0 T = 77 93.5 / 41.6, 5120 x 17408 Q6_K T = 256 235 /
+// 139, 4096 x 11008 Q8_0 T = 384 231 / 126. Its error against 64 bits is below gemmh's on each (1.4e-7 against 2.5e-7
+// for the first). Counted on the second: 118 vector instructions per wave and block, 64 of them the fma per element, and
+// 8 MFMAs, the matrix unit busy 34 % of the time.
 // Measured and not kept: the loads staged through registers (644 against 607 us), a ring of 4 one-block stages (623
 // against 617, 113 against 106), loads spread over the stage's arithmetic (738 against 735).
 template <int KIND, int NJ, int GR>
@@ -3895,8 +3896,8 @@ extern "C" __global__ __launch_bounds__(256) void amdc_gemv_q8_0_v16(const uint8
 // What bounds it is the issue of vector instructions, 1681 per wave and tile at T <= 8 where one product with columns
 // (quarter, token) for 4 tokens, whose halves met by DPP in half the lanes, took 3428; then a tile's chain of loads, two
 // waves per SIMD. Measured on MI355X (us, that form / this): T = 8 5120 x 17408 37.6 / 27.3, 17408 x 5120 38.0 / 29.9,
-// 4096 x 11008 24.8 / 17.9, 32000 x 4096 39.0 / 28.1, 152064 x 5120 221 / 164 (T = 2 182 / 157); T = 16 (one workgroup per
-// CU / two) 81 / 35, 87 / 37, 51 / 22, 97 / 35, 591 / 218.
+// 4096 x 11008 24.8 / 17.9, 32000 x 4096 39.0 / 28.1, 152064 x 5120 with the benchmark's weights 268-282 / 197-215; T = 16
+// (one workgroup per CU / two) 81 / 35, 87 / 37, 51 / 22, 97 / 35.
 template <int NH, int NS>
 __device__ __forceinline__ void gemv8_q6k_body(const uint8_t *__restrict__ W, const uint8_t *__restrict__ xq, float *__restrict__ y,
                                                u32 rows, u32 nb, const float *__restrict__ bias, const float *__restrict__ res, u32 T,

@@ -198,7 +198,7 @@ int amdc_gemv_q6k_x(const void *w, const float *x, float *y, uint32_t rows, uint
  * token, src/hip.c:1583-1588). Every vector's y equals the decode GEMV of that
  * vector (amdc_gemv_q4 / _q4k / _q8) bit for bit, at every K split, as the
  * reference's multi-token kernels equal its single-token one
- * (kernels/ie_kernels.c:481-482); Q6_K's agrees within the 1e-5 bound. */
+ * (kernels/ie_kernels.c:481-482); so does Q6_K's (amdc_gemv_q6k). */
 int amdc_gemv_q4_t(const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res,
                    uint32_t T, uint32_t xs, uint32_t ys, uint32_t rs, void *stream);
 int amdc_gemv_q4k_t(const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res,
@@ -216,7 +216,8 @@ int amdc_gemv_q6k_t(const void *w, const uint8_t *xq, float *y, uint32_t rows, u
  * sums of the sub-blocks are exact: by default on the f16 MFMA with the 6-bit
  * scale folded into the weights (q sc <= 945 and the int8 activations are f16
  * integers; every partial sum is an integer below 2^24; the min term on the bf16
- * MFMA from exact parts), or on the int8 MFMA (tuning); f32 outputs within 1e-5 of cpu_gemv_q4k per token row. Uses a
+ * MFMA from parts that are exact where |d_a asum| >= 2^-110), or on the int8 MFMA (tuning); f32 outputs within 1e-5 of
+ * cpu_gemv_q4k per token row (on matrices of more than 2^22 weights for d_a from 1e-36 up: below, bf16 ends). Uses a
  * device workspace that the library allocates on the first call of a size
  * (call once outside graph capture before capturing). */
 int amdc_gemm_q4k(const void *w, const uint8_t *xq, float *y, uint32_t rows, uint32_t nb, const float *bias, const float *res,
